@@ -1,0 +1,62 @@
+"""GPU parity of the attention's forms against the oracle: key counts around every change of form (scores
+kept by one, two or four waves, or recomputed; 64-key tiles with and without a remainder; more keys than
+fit the LDS constants at once), full and causal, with the integer arithmetic and with the general one
+(large shifts, or a table that starts below 2^30 or rises)."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from tests.conftest import assert_equal, to_np
+from tests.test_gpu_attention import dev, gpu_heads, gpu_v, host
+from vela_amd import attention as va
+
+pytestmark = pytest.mark.gpu
+
+EXP = oracle.exp_table()
+RISING = EXP[::-1].copy()          # not monotone falling: the general form
+SMALL = (EXP >> 8).copy()          # starts at 2^22: r needs more than 32 bits
+
+
+def check(B, heads, Tq, Tk, causal, scale=70000, table=EXP, seed=0, big_keys=False):
+    r = np.random.default_rng(seed + 1000 * Tq + Tk)
+    C = heads * 64
+    Tqp, Tkp = (Tq + 63) // 64 * 64, (Tk + 63) // 64 * 64
+    X = [r.normal(0, scale, (B * n, C)).astype(np.int32) for n in (Tq, Tk, Tk)]
+    X[0][::5] = (X[0][::5] * 0.01).astype(np.int32)      # other shifts among the rows
+    X[1][::7] = (X[1][::7] * 0.02).astype(np.int32)
+    if big_keys:
+        X[1][1] = 1 << 29                                 # eq + ek > 12 for every query
+    q, k, v = gpu_heads(X[0], B, Tq, C, heads, Tqp), gpu_heads(X[1], B, Tk, C, heads, Tkp), gpu_v(X[2], B, Tk, C, heads, Tkp)
+    out = torch.full((B * Tq, C), 0x5a5a5a5a, dtype=torch.int32, device="cuda")
+    rm = torch.zeros(B * Tq, dtype=torch.int32, device="cuda")
+    va.k_fused_attention(*q[:5], k[0], k[1], k[2], k[5], *v, B, heads, Tq, Tqp, Tk, Tkp, causal, dev(table), C, None, None, out, rm)
+    torch.cuda.synchronize()
+    qh, kh, vh = host(q), host(k), host(v)
+    wrm = np.zeros(B * Tq, np.uint32)
+    want = oracle.attention(qh[0], qh[1], qh[2], kh[0], kh[1], kh[2], vh[0], vh[1], vh[2], B, heads, Tq, Tqp, Tk, Tkp, causal, table, C, rowmax=wrm)
+    what = f"Tq {Tq} Tk {Tk} causal {causal}"
+    assert_equal(to_np(out), want, what + " out")
+    assert_equal(to_np(rm).view(np.uint32), wrm, what + " rowmax")
+
+
+@pytest.mark.parametrize("Tk", [1, 64, 65, 128, 129, 192, 256, 257, 448, 512, 513, 1000, 1024, 1025, 1217, 4096, 4161])
+def test_key_counts(gpu, Tk):
+    check(1, 2, 37, Tk, False)
+
+
+@pytest.mark.parametrize("T", [1, 17, 64, 130, 257, 300, 513, 700, 1100])
+def test_causal(gpu, T):
+    check(1, 2, T, T, True)
+
+
+@pytest.mark.parametrize("Tk", [77, 250, 400, 900, 1090])
+@pytest.mark.parametrize("kw", [dict(table=RISING), dict(table=SMALL), dict(big_keys=True)])
+def test_general_form(gpu, Tk, kw):
+    check(1, 1, 20, Tk, False, **kw)
+
+
+def test_dominant_key(gpu):
+    """One key takes a row's whole probability (sum of E = 2^30, r = 2^32, P = 32768 before the clamp)."""
+    for Tk in (3, 200, 1100):
+        check(1, 1, 33, Tk, False, scale=600000)
