@@ -1,7 +1,8 @@
 """GPU parity of the attention's forms against the oracle: key counts around every change of form (scores
 kept by one, two or four waves, or recomputed; 64-key tiles with and without a remainder; more keys than
 fit the LDS constants at once), full and causal, with the integer arithmetic and with the general one
-(large shifts, or a table that starts below 2^30 or rises)."""
+(large shifts, or a table that starts below 2^30 or rises); and the forms of the operand
+producers."""
 import numpy as np
 import pytest
 import torch
@@ -38,6 +39,47 @@ def check(B, heads, Tq, Tk, causal, scale=70000, table=EXP, seed=0, big_keys=Fal
     what = f"Tq {Tq} Tk {Tk} causal {causal}"
     assert_equal(to_np(out), want, what + " out")
     assert_equal(to_np(rm).view(np.uint32), wrm, what + " rowmax")
+
+
+def edge_rows(r, shape):
+    X = r.normal(0, 60000, shape).astype(np.int32)
+    X[:: 9] = r.integers(-(2**31), 2**31, X[::9].shape, dtype=np.int64).astype(np.int32)
+    X[3:: 11] = r.integers(-3, 4, X[3::11].shape)
+    X[5:: 50] = -(2**31)
+    return X
+
+
+@pytest.mark.parametrize("B,T,heads,C,Tp,shift", [(1, 1, 1, 64, 64, 0), (2, 77, 3, 192, 128, 0), (1, 50, 2, 130, 64, 0), (1, 50, 2, 128, 64, 1),
+                                                  (8, 1000, 5, 324, 1024, 0), (3, 33, 12, 768, 35, 0)])
+def test_quant_heads_forms(gpu, B, T, heads, C, Tp, shift):
+    """Aligned rows and planes, odd widths, a source off 16 bytes (shift elements), few and many rows."""
+    X = edge_rows(np.random.default_rng(T + C), (B * T, C))
+    flat = torch.zeros(B * T * C + 4, dtype=torch.int32, device="cuda")
+    Xd = flat[shift : shift + B * T * C]
+    Xd.copy_(dev(X).reshape(-1))
+    n = B * heads * Tp
+    got = [torch.full((n, 64), 0x5a, dtype=torch.int8, device="cuda") for _ in range(2)] + [torch.full((n,), 7, dtype=torch.int32, device="cuda")]
+    got += [torch.full((n,), 7, dtype=torch.int64, device="cuda") for _ in range(3)]
+    va.k_quant_heads(Xd, B, T, C, heads, Tp, *got)
+    torch.cuda.synchronize()
+    for g, w, name in zip(got, oracle.quant_heads(X, B, T, C, heads, Tp), ("hi", "lo", "e", "hs", "ls", "tsum")):
+        assert_equal(to_np(g), w, name)
+
+
+@pytest.mark.parametrize("B,Tk,heads,C,Tkp", [(1, 1, 1, 64, 64), (2, 64, 2, 128, 64), (2, 65, 2, 130, 128), (1, 100, 3, 192, 256), (2, 128, 1, 65, 128),
+                                              (2, 129, 2, 128, 192), (1, 700, 5, 320, 704)])
+def test_quant_v_forms(gpu, B, Tk, heads, C, Tkp):
+    """One block a group and rows split over blocks, remainders of both, twice into the same buffers."""
+    r = np.random.default_rng(Tk)
+    G = B * heads
+    got = [torch.full((G * 64, Tkp), 0x5a, dtype=torch.int8, device="cuda") for _ in range(2)]
+    got += [torch.full((G * 64,), 99, dtype=torch.int32, device="cuda"), torch.full((G * 64,), 99, dtype=torch.int64, device="cuda")]
+    for scale in (60000, 900):
+        X = (edge_rows(r, (B * Tk, C)) if scale > 1000 else r.normal(0, scale, (B * Tk, C)).astype(np.int32))
+        va.k_quant_v(dev(X), B, Tk, C, heads, Tkp, *got)
+        torch.cuda.synchronize()
+        for g, w, name in zip(got, oracle.quant_v(X, B, Tk, C, heads, Tkp), ("vthi", "vtlo", "ev", "vsum")):
+            assert_equal(to_np(g), w, name)
 
 
 @pytest.mark.parametrize("Tk", [1, 64, 65, 128, 129, 192, 256, 257, 448, 512, 513, 1000, 1024, 1025, 1217, 4096, 4161])

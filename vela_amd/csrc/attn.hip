@@ -646,6 +646,68 @@ __global__ void __launch_bounds__(256) quant_heads_kernel(const int32_t* __restr
     if (lane == 0) { e[w] = ee; hs[w] = sh; ls[w] = sl; tsum[w] = st; }
 }
 
+// The same with 16 lanes to a row, four values a lane and R rows of each 16-lane group in flight (rows R n +
+// i * 16 of a block): one 16-byte load and two 4-byte stores per lane and row, reductions inside a DPP row,
+// where the form above stores single bytes and shuffles through 64 lanes (8 x 1024 x 640 in 10 heads, 31 MB:
+// 26.3 -> 7.7 us). Needs a 16-byte aligned X, C % 4 == 0 and 4-byte aligned planes.
+template <int CTRL>
+__device__ __forceinline__ int dpp(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, false); }
+__device__ __forceinline__ uint32_t row16_umax(uint32_t v) {
+    v = max(v, uint32_t(dpp<0xB1>(int(v))));
+    v = max(v, uint32_t(dpp<0x4E>(int(v))));
+    v = max(v, uint32_t(dpp<0x141>(int(v))));
+    return max(v, uint32_t(dpp<0x140>(int(v))));
+}
+__device__ __forceinline__ int row16_sum(int v) {
+    v += dpp<0xB1>(v);
+    v += dpp<0x4E>(v);
+    v += dpp<0x141>(v);
+    return v + dpp<0x140>(v);
+}
+template <int R>
+__global__ void __launch_bounds__(256) quant_heads_vec_kernel(const int32_t* __restrict__ X, int B, int T, int C, int heads, int Tp,
+                                                              int8_t* __restrict__ hi, int8_t* __restrict__ lo, int32_t* __restrict__ e,
+                                                              long long* __restrict__ hs, long long* __restrict__ ls, long long* __restrict__ tsum) {
+    const int l16 = threadIdx.x & 15;
+    const unsigned w0 = blockIdx.x * (16 * R) + (threadIdx.x >> 4), rows = unsigned(B) * heads * Tp;   // below 2^31
+    int4 x[R];
+    bool real[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        const unsigned w = w0 + 16 * i;
+        const int g = int(w / unsigned(Tp)), t = int(w - unsigned(g) * Tp), b = g / heads, h = g - b * heads;
+        real[i] = w < rows && t < T;
+        x[i] = make_int4(0, 0, 0, 0);
+        if (real[i]) x[i] = *reinterpret_cast<const int4*>(X + (size_t(b) * T + t) * C + h * 64 + 4 * l16);
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        const unsigned w = w0 + 16 * i;
+        const int v[4] = {x[i].x, x[i].y, x[i].z, x[i].w};
+        const int ee = rowexp_u32(row16_umax(max(max(uabs(v[0]), uabs(v[1])), max(uabs(v[2]), uabs(v[3])))));
+        unsigned h4 = 0, l4 = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int q = quant16_32(v[j], ee);
+            h4 |= unsigned(q >> 8 & 255) << (8 * j);
+            l4 |= unsigned((q & 255) ^ 128) << (8 * j);
+        }
+        const int sh = row16_sum(__builtin_amdgcn_sdot4(int(h4), 0x01010101, 0, false));
+        const int sl = row16_sum(__builtin_amdgcn_sdot4(int(l4), 0x01010101, 0, false));
+        if (w < rows) {   // a pad row is the value 0: hi 0, lo -128
+            const size_t o = size_t(w) * 16 + l16;
+            reinterpret_cast<unsigned*>(hi)[o] = h4;
+            reinterpret_cast<unsigned*>(lo)[o] = l4;
+            if (l16 == 0) {
+                e[w] = ee;
+                hs[w] = sh;
+                ls[w] = sl;
+                tsum[w] = 256 * sh + sl + 128 * 64;
+            }
+        }
+    }
+}
+
 // src/kernels.cu:799-805: rows t in [T, Tp) of every group take the value 0
 __global__ void __launch_bounds__(256) quant_heads_pad_kernel(int G, int T, int Tp, int8_t* __restrict__ hi, int8_t* __restrict__ lo, int32_t* __restrict__ e,
                                                               long long* __restrict__ hs, long long* __restrict__ ls, long long* __restrict__ tsum) {
@@ -659,65 +721,93 @@ __global__ void __launch_bounds__(256) quant_heads_pad_kernel(int G, int T, int 
     if (lane == 0) { e[row] = 0; hs[row] = 0; ls[row] = -128 * 64; tsum[row] = 0; }
 }
 
-// src/kernels.cu:632-650 (k_quant_v, exponents): one block per group, thread (d, slice) scanning
-// rows slice, slice + 4, ...; ev = row_exp(max |x|) per dimension; vsum cleared for the write pass
-__global__ void __launch_bounds__(256) quant_v_exp_kernel(const int32_t* __restrict__ X, int Tk, int C, int heads, int32_t* __restrict__ ev,
-                                                          long long* __restrict__ vsum) {
+// src/kernels.cu:632-650 (k_quant_v, exponents): ev = row_exp(max |x|) per dimension. row_exp is monotone,
+// so blocks of QV_ROWS rows of a group combine their exponents by an atomic maximum on a cleared ev; the
+// clear also zeroes vsum for the write pass. One block per group scanning all rows, four loads deep, took
+// 267 us of 4096 rows in 40 groups (1 MB a block); in runs of 128 rows the clear and the scan take 11.
+constexpr int QV_ROWS = 128;
+constexpr int QV_ONE = 128;    // keys a block quantises on its own, in one launch in place of three
+__global__ void __launch_bounds__(256) quant_v_clear_kernel(int n, int32_t* __restrict__ ev, long long* __restrict__ vsum) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) {
+        ev[i] = 0;
+        vsum[i] = 0;
+    }
+}
+__global__ void __launch_bounds__(256) quant_v_exp_kernel(const int32_t* __restrict__ X, int Tk, int C, int heads, int32_t* __restrict__ ev) {
     __shared__ uint32_t s_m[4][64];
-    const int g = blockIdx.x, b = g / heads, h = g - b * heads, d = threadIdx.x & 63, sl = threadIdx.x >> 6;
+    const int g = blockIdx.y, b = g / heads, h = g - b * heads, d = threadIdx.x & 63, sl = threadIdx.x >> 6;
+    const int t0 = blockIdx.x * QV_ROWS + sl;
     const int32_t* x = X + size_t(b) * Tk * C + h * 64 + d;
     uint32_t m = 0;
-    for (int t = sl; t < Tk; t += 4) m = max(m, uabs(x[size_t(t) * C]));
+#pragma unroll 8
+    for (int i = 0; i < QV_ROWS; i += 4) m = max(m, uabs(x[size_t(min(t0 + i, Tk - 1)) * C]));
     s_m[sl][d] = m;
     __syncthreads();
     if (sl == 0) {
         m = max(max(s_m[0][d], s_m[1][d]), max(s_m[2][d], s_m[3][d]));
-        ev[g * 64 + d] = rowexp_u32(m);
-        vsum[g * 64 + d] = 0;
+        const int e = rowexp_u32(m);
+        if (e) atomicMax(ev + g * 64 + d, e);
     }
 }
 
 // src/kernels.cu:651-672 (k_quant_v, transposed write): block per (64-row tile, group): the tile in
 // LDS, then thread (d, quarter) quantises 16 consecutive rows of dimension d, writes them as 16
 // bytes of each plane of vt[g * 64 + d], and adds its part of vsum
+// ONE: the block has all of its group's rows (Tkp <= QV_ONE), finds the exponents itself and writes ev and vsum.
+template <bool ONE>
 __global__ void __launch_bounds__(256) quant_v_write_kernel(const int32_t* __restrict__ X, int Tk, int C, int heads, int Tkp,
-                                                            const int32_t* __restrict__ ev, int8_t* __restrict__ vth, int8_t* __restrict__ vtl,
+                                                            int32_t* __restrict__ ev, int8_t* __restrict__ vth, int8_t* __restrict__ vtl,
                                                             long long* __restrict__ vsum) {
-    __shared__ int32_t tile[64][65];
-    __shared__ long long s_s[4][64];
+    constexpr int NT = ONE ? QV_ONE / 64 : 1;   // tiles of the block
+    __shared__ int32_t tile[NT * 64][65];
+    __shared__ int s_e[4][64];
     const int g = blockIdx.y, t0 = blockIdx.x * 64, b = g / heads, h = g - b * heads;
     const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    for (int r = ty; r < 64; r += 4) {
-        const int t = t0 + r;
-        tile[r][tx] = t < Tk ? X[(size_t(b) * Tk + t) * C + h * 64 + tx] : 0;
+    const int32_t* x = X + size_t(b) * Tk * C + h * 64 + tx;
+    uint32_t m = 0;
+#pragma unroll
+    for (int r = 0; r < NT * 64; r += 4) {
+        const int t = t0 + r + ty;
+        const int v = t < Tk ? x[size_t(t) * C] : 0;
+        tile[r + ty][tx] = v;
+        m = max(m, uabs(v));
     }
+    if (ONE) s_e[ty][tx] = rowexp_u32(m);
     __syncthreads();
     const int d = threadIdx.x >> 2, qt = threadIdx.x & 3;
-    const int e = ev[g * 64 + d];
-    unsigned hw[4], lw[4];
-    long long s = 0;
+    const int e = ONE ? max(max(s_e[0][d], s_e[1][d]), max(s_e[2][d], s_e[3][d])) : ev[g * 64 + d];
+    int s = 0;   // of 16 NT values below 2^15
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        unsigned hv = 0, lv = 0;
+    for (int k = 0; k < NT; ++k) {
+        if (ONE && k * 64 >= Tkp) break;
+        unsigned hw[4], lw[4];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int r = 16 * qt + 4 * c + k;
-            const int q = t0 + r < Tk ? quant16_32(tile[r][d], e) : 0;
-            s += q;
-            hv |= unsigned(q >> 8 & 255) << (8 * k);
-            lv |= unsigned(((q & 255) - 128) & 255) << (8 * k);
+        for (int c = 0; c < 4; ++c) {
+            unsigned hv = 0, lv = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int q = quant16_32(tile[64 * k + 16 * qt + 4 * c + i][d], e);   // rows past Tk hold 0
+                s += q;
+                hv |= unsigned(q >> 8 & 255) << (8 * i);
+                lv |= unsigned((q & 255) ^ 128) << (8 * i);
+            }
+            hw[c] = hv;
+            lw[c] = lv;
         }
-        hw[c] = hv;
-        lw[c] = lv;
+        const size_t o = (size_t(g) * 64 + d) * Tkp + t0 + 64 * k + 16 * qt;
+        *reinterpret_cast<v4i*>(vth + o) = v4i{int(hw[0]), int(hw[1]), int(hw[2]), int(hw[3])};
+        *reinterpret_cast<v4i*>(vtl + o) = v4i{int(lw[0]), int(lw[1]), int(lw[2]), int(lw[3])};
     }
-    const size_t o = (size_t(g) * 64 + d) * Tkp + t0 + 16 * qt;
-    *reinterpret_cast<v4i*>(vth + o) = v4i{int(hw[0]), int(hw[1]), int(hw[2]), int(hw[3])};
-    *reinterpret_cast<v4i*>(vtl + o) = v4i{int(lw[0]), int(lw[1]), int(lw[2]), int(lw[3])};
-    s_s[qt][d] = s;
-    __syncthreads();
-    if (threadIdx.x < 64) {
-        const long long t = s_s[0][threadIdx.x] + s_s[1][threadIdx.x] + s_s[2][threadIdx.x] + s_s[3][threadIdx.x];
-        atomicAdd(reinterpret_cast<unsigned long long*>(vsum + g * 64 + threadIdx.x), (unsigned long long)t);
+    s += dpp<0xB1>(s);   // the four quarters of a dimension are a quad of lanes
+    s += dpp<0x4E>(s);
+    if (qt == 0) {
+        if (ONE) {
+            ev[g * 64 + d] = e;
+            vsum[g * 64 + d] = s;
+        } else {
+            atomicAdd(reinterpret_cast<unsigned long long*>(vsum + g * 64 + d), (unsigned long long)(long long)s);
+        }
     }
 }
 
@@ -744,7 +834,11 @@ hipError_t launch_attention(hipStream_t st, const AttnArgs& a, int G) {
 hipError_t launch_quant_heads(hipStream_t st, const int32_t* X, int B, int T, int C, int heads, int Tp, int8_t* hi, int8_t* lo, int32_t* e, long long* hs,
                               long long* ls, long long* tsum) {
     const long long rows = (long long)B * heads * Tp;
-    hipLaunchKernelGGL(quant_heads_kernel, dim3(unsigned((rows + 3) / 4)), dim3(256), 0, st, X, B, T, C, heads, Tp, hi, lo, e, hs, ls, tsum);
+    const uintptr_t al = reinterpret_cast<uintptr_t>(X) % 16 | reinterpret_cast<uintptr_t>(hi) % 4 | reinterpret_cast<uintptr_t>(lo) % 4 | unsigned(C % 4);
+    if (al || rows > INT_MAX - 64) hipLaunchKernelGGL(quant_heads_kernel, dim3(unsigned((rows + 3) / 4)), dim3(256), 0, st, X, B, T, C, heads, Tp, hi, lo, e, hs, ls, tsum);
+    // few rows: one per 16-lane group, so that every CU has a block
+    else if (rows < 32768) hipLaunchKernelGGL(quant_heads_vec_kernel<1>, dim3(unsigned((rows + 15) / 16)), dim3(256), 0, st, X, B, T, C, heads, Tp, hi, lo, e, hs, ls, tsum);
+    else hipLaunchKernelGGL(quant_heads_vec_kernel<4>, dim3(unsigned((rows + 63) / 64)), dim3(256), 0, st, X, B, T, C, heads, Tp, hi, lo, e, hs, ls, tsum);
     return hipGetLastError();
 }
 
@@ -756,8 +850,13 @@ hipError_t launch_quant_heads_pad(hipStream_t st, int G, int T, int Tp, int8_t* 
 
 hipError_t launch_quant_v(hipStream_t st, const int32_t* X, int B, int Tk, int C, int heads, int Tkp, int8_t* vth, int8_t* vtl, int32_t* ev, long long* vsum) {
     const int G = B * heads;
-    hipLaunchKernelGGL(quant_v_exp_kernel, dim3(unsigned(G)), dim3(256), 0, st, X, Tk, C, heads, ev, vsum);
-    hipLaunchKernelGGL(quant_v_write_kernel, dim3(unsigned(Tkp / 64), unsigned(G)), dim3(256), 0, st, X, Tk, C, heads, Tkp, ev, vth, vtl, vsum);
+    if (Tkp <= QV_ONE) {
+        hipLaunchKernelGGL(quant_v_write_kernel<true>, dim3(1, unsigned(G)), dim3(256), 0, st, X, Tk, C, heads, Tkp, ev, vth, vtl, vsum);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(quant_v_clear_kernel, dim3(unsigned((G * 64 + 255) / 256)), dim3(256), 0, st, G * 64, ev, vsum);
+    hipLaunchKernelGGL(quant_v_exp_kernel, dim3(unsigned((Tk + QV_ROWS - 1) / QV_ROWS), unsigned(G)), dim3(256), 0, st, X, Tk, C, heads, ev);
+    hipLaunchKernelGGL(quant_v_write_kernel<false>, dim3(unsigned(Tkp / 64), unsigned(G)), dim3(256), 0, st, X, Tk, C, heads, Tkp, ev, vth, vtl, vsum);
     return hipGetLastError();
 }
 

@@ -1110,7 +1110,7 @@ int vgemm_quant_heads_pad(void* stream, int G, int T, int Tp, int8_t* hi, int8_t
 
 int vgemm_quant_v(void* stream, const int32_t* X, int B, int Tk, int C, int heads, int Tkp, int8_t* vthi, int8_t* vtlo, int32_t* ev, int64_t* vsum,
                   uint32_t* scratch) {
-    (void)scratch;   // the column maxima stay inside one block per group here
+    (void)scratch;   // the exponents combine in ev itself
     if (!X || !vthi || !vtlo || !ev || !vsum || B <= 0 || heads <= 0 || Tk <= 0 || Tkp < Tk || C < 64 * heads)
         return fail(VGEMM_ERR_ARG, "quant_v: bad arguments");
     if (Tkp % 64 || !aligned16(vthi) || !aligned16(vtlo)) return fail(VGEMM_ERR_ARG, "quant_v: Tkp %% 64 == 0 and 16-byte aligned planes required");
