@@ -180,8 +180,11 @@ void stripe_ranges(const vk::GemmParams& p, int& cs, int& kper) {
     cs = cdiv(nch, kper);
 }
 
-// Automatic use, with no per-row shifts (rows with e != 0 leave the kernels' integer epilogue for
-// their slow int64 form; the tile kernels cover them):
+// Automatic use. Calls with per-row shifts run the sixteen-row kernel's form for them, PLAIN too (32768 x 320
+// with row shifts: x 2560 GEGLU 118.3 -> 66.4 us, x 320 PLAIN 20.4 -> 16.9, 16384 x 320 x 1280 GELU 39.7 ->
+// 25.4, against the tile kernels), by the last rule below alone (3096 x 320 x 2560, 980 tiles, 18.3 -> 16.9;
+// below it the tile kernels stay ahead: 16384 x 320 x 320, 768 tiles, 12.3 against 13.4, 1400 x 320 x 2560,
+// 440 tiles, 10.9 against 14.7) and not with a residual, which that kernel does not add. Without shifts:
 //  * many rows (a block keeps its rows in registers and streams its columns, so the kernels need a
 //    few hundred row stripes to fill the GPU); residual calls qualify, the kernel loading a batch's
 //    residuals ahead of its arithmetic (UNet 32768 x 320 x 320 residual layers: 23.1 us against
@@ -196,8 +199,8 @@ void stripe_ranges(const vk::GemmParams& p, int& cs, int& kper) {
 //    20.0 -> 16.0, 8192 x 160 x 1280 PLAIN 18.1 -> 13.2, with a residual 8192 x 320 x 1280
 //    29.4 -> 21.1, 960 tiles 4-16 % faster; at 640 and 768 tiles the tile kernels stay ahead,
 //    4096 x 320 x 1280 PLAIN 11.2 against 12.1 us).
-bool stripe_auto(const vk::GemmParams& p) {
-    if (p.e) return false;
+bool stripe_auto(int epi, const vk::GemmParams& p) {
+    if (p.e) return !p.R && p.Mreal >= 1024 && (long long)cdiv(p.Mreal, 64) * cdiv(p.Nreal, 128) >= 15LL * NCU / 4;
     if (cdiv(p.Mreal, STRIPE_BM) >= 2 * NCU / 4 && p.Mreal >= 16384) return true;
     if (p.Mreal >= 1024 && (long long)cdiv(p.Mreal, 64) * cdiv(p.Nreal, 128) >= 15LL * NCU / 4) return true;
     int cs, kper;
@@ -644,11 +647,11 @@ int hl2_impl(void* stream, const VgemmASrc* A, int Mp, int Mreal, const int8_t* 
 
     // shallow GEMMs with many rows: the row-stationary kernel (forced by variant 4 where it applies)
     if (stripe_applies(A->src, epi, p) && !p.gnstat &&
-        (g_variant == VARIANT_STRIPE || g_variant == VARIANT_STRIPE16 || (g_variant < 0 && stripe_auto(p)))) {
+        (g_variant == VARIANT_STRIPE || g_variant == VARIANT_STRIPE16 || (g_variant < 0 && stripe_auto(epi, p)))) {
         const int nout = epi == VGEMM_EPI_GEGLU ? Nreal / 2 : Nreal;
         p.y_bytes = unsigned(((long long)(Mreal - 1) * E->ldy + nout) * 4);
         stripe_grid(p);
-        const bool s16 = !p.R && (g_variant == VARIANT_STRIPE16 || (g_variant < 0 && stripe16_auto(epi)));
+        const bool s16 = !p.R && (g_variant == VARIANT_STRIPE16 || (g_variant < 0 && (stripe16_auto(epi) || p.e)));
         if (s16) return hip_status(vk::launch_stripe16(A->src, epi, p, st), "gemm_hl stripe launch");
         return hip_status(vk::launch_stripe(A->src, epi, p, st), "gemm_hl stripe launch");
     }

@@ -22,7 +22,10 @@
 // chunks of sums in registers: waves 0..3 run a chunk's MFMAs (four subtiles x five K steps x two
 // planes) and then its requantising epilogue, waves 4..7 the previous chunk's epilogue and then the
 // chunk's MFMAs, the plane sums folded into one int32 per element (256 Chi + Clo, exact for
-// Kp <= 320) across the barrier. The int64 form (per-row shifts, columns whose constants fail the
+// Kp <= 320) across the barrier. RX instantiations take rows with shifts in the integer form too (the planes
+// the norms and row quantisations write): the multiplier is shifted by the row's e and the offset term added
+// to the sum, two more instructions per requantisation (32768 x 320 x 2560 GEGLU with row shifts: 118 us on
+// the 128x128 tiles, 66-68 here, 62 without shifts). The int64 form (per-row shifts, columns whose constants fail the
 // integer form's bounds, tables outside [0, 65536]) runs a plain loop, a chunk's MFMAs then its
 // outputs element by element.
 #pragma once
@@ -40,7 +43,7 @@ struct Stripe16Cfg {
     static_assert(WR == 16 && NKS * 64 == 32 * StripeCfg::NKS, "stripe16 geometry");
 };
 
-template <int SRC, int EPI>
+template <int SRC, int EPI, bool RX>
 __global__ void __launch_bounds__(512, 4) stripe16_kernel(const GemmParams p) {
     using S = StripeCfg;
     using G = Stripe16Cfg;
@@ -124,7 +127,7 @@ __global__ void __launch_bounds__(512, 4) stripe16_kernel(const GemmParams p) {
     vm_wait<AL>();   // the column constants, the table and chunk cb's W (older than the row loads)
     block_barrier();
     bool lut_ok;
-    const int form = stripe_setup<EPI, NT>(p, sh, tid, m0, cb, ncols, craw, erv, L2048, lut_ok);
+    const int form = stripe_setup<EPI, NT, RX>(p, sh, tid, m0, cb, ncols, craw, erv, L2048, lut_ok);
 
     // ---- the rows' hi/lo split (int16 rows), once they have arrived
     if constexpr (SRC == SRC_I16) {
@@ -150,9 +153,30 @@ __global__ void __launch_bounds__(512, 4) stripe16_kernel(const GemmParams p) {
         return *reinterpret_cast<const v4i*>(sW + t * S::KSTEP + pswz(16 * u + fr, fg));
     };
 
-    if (form == FORM_INT) {
-        // ---- chunk loop of the integer form
+    if (form != FORM_EXACT) {
+        // ---- chunk loop of the integer form (RX: and of the form in double)
         int X[NSUB][4];   // a chunk's folded sums 256 Chi + Clo
+        unsigned e4 = 0;  // RX: the shifts of the lane's four rows, one a byte
+        if constexpr (RX) {
+            const int* er = sh.erow + wave * G::WR + 4 * fg;
+            e4 = unsigned(er[0] & 255) | unsigned(er[1] & 255) << 8 | unsigned(er[2] & 255) << 16 | unsigned(er[3] & 255) << 24;
+        }
+        // requantisation of row v's sum A with the table entry at index j (RX: all of the entry)
+        struct Col { int4 k; };
+        auto col_at = [&](int j) __attribute__((always_inline)) {
+            if constexpr (RX) return Col{sh.tab[j]};
+            const StripeK3 k = stripe_tab3(sh.tab, j);
+            return Col{make_int4(k.m, k.lo, k.hi, 0)};
+        };
+        auto req_hi = [&](int A, const Col& c, int v, auto fp) __attribute__((always_inline)) {
+            if constexpr (decltype(fp)::value) {
+                return stripe_req_fp(A, c.k, int(e4 >> (8 * v) & 255u));
+            } else if constexpr (RX) {
+                return v == 0 ? stripe_req_rx<0>(A, c.k, e4) : v == 1 ? stripe_req_rx<1>(A, c.k, e4) : v == 2 ? stripe_req_rx<2>(A, c.k, e4) : stripe_req_rx<3>(A, c.k, e4);
+            } else {
+                return stripe_req_hi(A, StripeK3{c.k.x, c.k.y, c.k.z});
+            }
+        };
         struct EpiC { int4 ka[NOUT], kg[NOUT]; unsigned vbase[NOUT]; };
         // per-chunk constants of the epilogue of the chunk held in X: table entries of the lane's
         // columns and the byte offset of its first output (OOB past the output's columns)
@@ -168,18 +192,18 @@ __global__ void __launch_bounds__(512, 4) stripe16_kernel(const GemmParams p) {
             return k;
         };
         // output o = 4 u + v of the chunk held in X (PLAIN, GELU): requantise, store, row maximum
-        auto epi_one = [&](const EpiC& k, int o, auto rmax, auto full) __attribute__((always_inline)) {
+        auto epi_one = [&](const EpiC& k, int o, auto rmax, auto full, auto fp) __attribute__((always_inline)) {
             constexpr bool RMAX = decltype(rmax)::value, FULL = decltype(full)::value;
             const int u = o >> 2, v = o & 3;
             int y;
             unsigned ay;
             if constexpr (EPI == EPI_GELU) {
-                const int ya = stripe_req<NEEDLUT>(X[u][v], k.ka[u]);
+                const int ya = RX ? req_hi(X[u][v], Col{k.ka[u]}, v, fp) : stripe_req<NEEDLUT>(X[u][v], k.ka[u]);
                 unsigned h0;
                 y = stripe_mulsh16(ya, stripe_phi(sh.lut, ya), h0);
                 ay = unsigned(max(y, int(0u - unsigned(y))));
             } else {
-                y = stripe_req<NEEDLUT>(X[u][v], k.ka[u]);
+                y = RX ? req_hi(X[u][v], Col{k.ka[u]}, v, fp) : stripe_req<NEEDLUT>(X[u][v], k.ka[u]);
                 ay = unsigned(max(y, int(0u - unsigned(y))));
             }
             const unsigned soff = unsigned(v) * ldy4;
@@ -192,13 +216,13 @@ __global__ void __launch_bounds__(512, 4) stripe16_kernel(const GemmParams p) {
         // a product outside that range to a second pass that stores the saturated values again
         // (a lane's stores to one address stay in order). The row maximum then follows from each
         // row's max and min of y.
-        auto epilogue_geglu = [&](int tb, int ocol0, auto rmax, auto full) __attribute__((always_inline)) {
+        auto epilogue_geglu = [&](int tb, int ocol0, auto rmax, auto full, auto fp) __attribute__((always_inline)) {
             constexpr bool RMAX = decltype(rmax)::value, FULL = decltype(full)::value;
             int yv[NO];
 #pragma unroll
             for (int u = 0; u < NOUT; ++u) {
                 // the lane's a and g table entries and output offset for this subtile pair
-                const StripeK3 ka = stripe_tab3(sh.tab, tb + 16 * u + fr), kg = stripe_tab3(sh.tab, tb + CH / 2 + 16 * u + fr);
+                const Col ka = col_at(tb + 16 * u + fr), kg = col_at(tb + CH / 2 + 16 * u + fr);
                 const int ncol = ocol0 + 16 * u + fr;
                 const unsigned vbase = ncol < nlim ? rowoff + unsigned(ncol) * 4u : OOB;
                 auto store = [&](int y, int v) __attribute__((always_inline)) {
@@ -208,10 +232,10 @@ __global__ void __launch_bounds__(512, 4) stripe16_kernel(const GemmParams p) {
                 int hv[4];
 #pragma unroll
                 for (int v = 0; v < 4; ++v) {
-                    const int yg = stripe_req_hi(X[u + NSUB / 2][v], kg);
+                    const int yg = req_hi(X[u + NSUB / 2][v], kg, v, fp);
                     unsigned h0, hi;
                     const int ge = stripe_mulsh16(yg, stripe_phi(sh.lut, yg), h0);
-                    yv[4 * u + v] = stripe_mulsh16(stripe_req_hi(X[u][v], ka), ge, hi);
+                    yv[4 * u + v] = stripe_mulsh16(req_hi(X[u][v], ka, v, fp), ge, hi);
                     hv[v] = int(hi);
                     store(yv[4 * u + v], v);
                 }
@@ -235,13 +259,13 @@ __global__ void __launch_bounds__(512, 4) stripe16_kernel(const GemmParams p) {
                 }
             }
         };
-        auto epilogue = [&](int tb, int ocol0, auto rmax, auto full) __attribute__((always_inline)) {
+        auto epilogue = [&](int tb, int ocol0, auto rmax, auto full, auto fp) __attribute__((always_inline)) {
             if constexpr (GEGLU) {
-                epilogue_geglu(tb, ocol0, rmax, full);
+                epilogue_geglu(tb, ocol0, rmax, full, fp);
             } else {
                 const EpiC k = epi_consts(tb, ocol0);
 #pragma unroll
-                for (int o = 0; o < NO; ++o) epi_one(k, o, rmax, full);
+                for (int o = 0; o < NO; ++o) epi_one(k, o, rmax, full, fp);
             }
         };
         // the MFMAs of the chunk in LDS stage `stage`, two subtiles at a time (four independent
@@ -274,7 +298,7 @@ __global__ void __launch_bounds__(512, 4) stripe16_kernel(const GemmParams p) {
         // (their sums wait in X across the barrier), so that while one keeps the matrix core busy
         // the other works the VALU.
         const bool lagging = wave >= 4;
-        auto run = [&](auto rmax, auto full) __attribute__((always_inline)) {
+        auto run = [&](auto rmax, auto full, auto fp) __attribute__((always_inline)) {
             for (int c = cb; c < ce; ++c) {
                 prio_step(c);
                 const int stage = (c - cb) & 1;
@@ -287,19 +311,21 @@ __global__ void __launch_bounds__(512, 4) stripe16_kernel(const GemmParams p) {
                     block_barrier();
                 }
                 if (c + 1 < ce) issue(c + 1, stage ^ 1);
-                if (lagging && c > cb) epilogue((c - 1 - cb) * CH, GEGLU ? (c - 1) * (CH / 2) : (c - 1) * CH, rmax, full);
+                if (lagging && c > cb) epilogue((c - 1 - cb) * CH, GEGLU ? (c - 1) * (CH / 2) : (c - 1) * CH, rmax, full, fp);
                 mfma_chunk(stage);
-                if (!lagging) epilogue((c - cb) * CH, GEGLU ? c * (CH / 2) : c * CH, rmax, full);
+                if (!lagging) epilogue((c - cb) * CH, GEGLU ? c * (CH / 2) : c * CH, rmax, full, fp);
             }
-            if (lagging) epilogue((ce - 1 - cb) * CH, GEGLU ? (ce - 1) * (CH / 2) : (ce - 1) * CH, rmax, full);
+            if (lagging) epilogue((ce - 1 - cb) * CH, GEGLU ? (ce - 1) * (CH / 2) : (ce - 1) * CH, rmax, full, fp);
         };
         const bool full = m0 + BM <= p.Mreal;
-        if (p.rowmax) {
-            if (full) run(std::true_type{}, std::true_type{});
-            else run(std::true_type{}, std::false_type{});
+        if (RX && form == FORM_FP) {
+            run(std::true_type{}, std::false_type{}, std::bool_constant<RX>{});
+        } else if (p.rowmax) {
+            if (full) run(std::true_type{}, std::true_type{}, std::false_type{});
+            else run(std::true_type{}, std::false_type{}, std::false_type{});
         } else {
-            if (full) run(std::false_type{}, std::true_type{});
-            else run(std::false_type{}, std::false_type{});
+            if (full) run(std::false_type{}, std::true_type{}, std::false_type{});
+            else run(std::false_type{}, std::false_type{}, std::false_type{});
         }
         if (p.rowmax) {
             // lanes with the same fg hold the same four rows: reduce over the 16 columns, one atomic per row
@@ -370,13 +396,13 @@ __global__ void __launch_bounds__(512, 4) stripe16_kernel(const GemmParams p) {
     }
 }
 
-template <int SRC>
+template <int SRC, bool RX>
 hipError_t launch_stripe16_t(int epi, const GemmParams& p, hipStream_t st) {
     const dim3 grid(unsigned(p.mtiles * p.ntiles));
     switch (epi) {
-    case EPI_PLAIN: hipLaunchKernelGGL((stripe16_kernel<SRC, EPI_PLAIN>), grid, dim3(Stripe16Cfg::NT), 0, st, p); break;
-    case EPI_GEGLU: hipLaunchKernelGGL((stripe16_kernel<SRC, EPI_GEGLU>), grid, dim3(Stripe16Cfg::NT), 0, st, p); break;
-    case EPI_GELU: hipLaunchKernelGGL((stripe16_kernel<SRC, EPI_GELU>), grid, dim3(Stripe16Cfg::NT), 0, st, p); break;
+    case EPI_PLAIN: hipLaunchKernelGGL((stripe16_kernel<SRC, EPI_PLAIN, RX>), grid, dim3(Stripe16Cfg::NT), 0, st, p); break;
+    case EPI_GEGLU: hipLaunchKernelGGL((stripe16_kernel<SRC, EPI_GEGLU, RX>), grid, dim3(Stripe16Cfg::NT), 0, st, p); break;
+    case EPI_GELU: hipLaunchKernelGGL((stripe16_kernel<SRC, EPI_GELU, RX>), grid, dim3(Stripe16Cfg::NT), 0, st, p); break;
     default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

@@ -70,7 +70,9 @@ struct StripeCfg {
 template <bool LUT>
 struct StripeShared {
     unsigned char w[2][StripeCfg::STAGE];
-    int4 tab[StripeCfg::NCOLS];   // per column {m, C lo, C hi, s} of the integer form (GELU/GEGLU: m and C times 2^(32-s))
+    // per column {m, C lo, C hi, s} of the integer form (GELU/GEGLU: m and C times 2^(32-s); with row shifts
+    // {m 2^(32-s), 2^31, b, 128 wsum})
+    int4 tab[StripeCfg::NCOLS];
     // lut[i + 1] = (1024 L[i] - d 1024 (i - 1024) mod 2^32, d = L[i+1] - L[i]); lut[0] below, lut[2049]
     // above the table: 1024 phi(x) = lut[j].x + lut[j].y x (mod 2^32) for x in entry j's range
     int2 lut[LUT ? 2050 : 1];
@@ -81,7 +83,7 @@ struct StripeShared {
 // byte offset inside sh.lut of the raw table as the DMA delivers it (entries 0..2047)
 constexpr unsigned STRIPE_LUT_RAW = 8192;
 
-enum { FORM_INT = 0, FORM_EXACT = 1 };
+enum { FORM_INT = 0, FORM_EXACT = 1, FORM_FP = 2 };
 
 // ---- block set-up shared by the row-stationary kernels (NT threads per block, at least BM)
 
@@ -127,7 +129,13 @@ __device__ __forceinline__ void stripe_lut_dma(const GemmParams& p, StripeShared
 // LDS word per wave carry the result through the barrier that the table expansion needs anyway.
 // lut_ok: the table lies in [0, 65536] (the expanded table in LDS is then valid). Ends with a
 // block-wide barrier after the tables are written.
-template <int EPI, int NT>
+// RX (rows with shifts 0 <= e): y = floor((acc m 2^e + 2^(s-1)) / 2^s) + b, the high word of acc (m 2^(32-s)
+// << e) + b 2^32 + 2^31. The bounds above then hold with |m| 2^e for |m|: each column gives the largest e it
+// allows (2 |m| 2^e < 2^s and Kp |m| 2^e < 2^(8+s), from bit lengths), each wave's smallest and the block's
+// largest e meet in the same LDS words. A model's columns (m < 2^15, s about 24) allow e up to 8. Blocks past
+// those bounds take the form in double (FORM_FP) when |m| Kp < 2^30 and 1 <= s - e, s <= 52: acc m is then below
+// 2^53, floor(fma(acc, m 2^(e-s), 1/2)) is exact, and its conversion and the add of b saturate.
+template <int EPI, int NT, bool RX = false>
 __device__ __forceinline__ int stripe_setup(const GemmParams& p, StripeShared<EPI == EPI_GEGLU || EPI == EPI_GELU>& sh, int tid,
                                             int m0, int cb, int ncols, const v4i* craw, int erv, int L2048, bool& lut_ok) {
     constexpr bool NEEDLUT = EPI == EPI_GEGLU || EPI == EPI_GELU;
@@ -155,6 +163,9 @@ __device__ __forceinline__ int stripe_setup(const GemmParams& p, StripeShared<EP
     const unsigned mlim = (1u << 30) / unsigned(p.Kp);   // |m| < mlim  <=>  |m| Kp < 2^30
     int4 cc[CPT];
     bool bad = false;
+    int eallow = 31, emax = 0;        // RX
+    int eallow_fp = 31;
+    bool bad_fp = false;
 #pragma unroll
     for (int q = 0; q < CPT; ++q) {
         const int j = tid + NT * q;
@@ -170,19 +181,55 @@ __device__ __forceinline__ int stripe_setup(const GemmParams& p, StripeShared<EP
         // GELU/GEGLU: 2 |m| < 2^s, so that m 2^(32-s) fits in int32: the table then holds the
         // multiplier and the constant pre-shifted by 32 - s and the result is the high word of the
         // product (s = 0 passes with m = 0 only, as in the unused slots)
+        if constexpr (RX) {
+            const int la = 32 - __clz(int(am)), lk = 32 - __clz(int(am * unsigned(p.Kp)));   // bit lengths (am < mlim)
+            const bool both = am < mlim && uabs(c.w) <= 128u * unsigned(p.Kp);
+            bad |= !(sok && both && uabs(c.z) < (1u << 30));
+            bad_fp |= !(both && unsigned(c.y) <= 52u);
+            if (am) {
+                eallow = min(eallow, min(c.y - 1 - la, 8 + c.y - lk));
+                eallow_fp = min(eallow_fp, c.y - 1);
+            } else if (live && c.y < 1) {
+                eallow_fp = -1;   // s = 0 with m = 0: left to the general form
+            }
+            continue;
+        }
         const bool hiok = !NEEDLUT || (sok && (u64(am) << 1) < (u64(1) << c.y));
         bad |= !(sok && umok && hiok && uabs(c.w) <= 128u * unsigned(p.Kp) && uabs(c.z) < (1u << 30));
     }
     if (tid < BM) {
         sh.erow[tid] = erv;
-        bad |= m0 + tid < p.Mreal && erv != 0;
+        if constexpr (RX) {
+            if (m0 + tid < p.Mreal) {
+                bad |= erv < 0;
+                bad_fp |= erv < 0;
+                emax = min(max(erv, 0), 63);
+            }
+        } else {
+            bad |= m0 + tid < p.Mreal && erv != 0;
+        }
+    }
+    if constexpr (RX) {
+        eallow = max(wave_min_i32(eallow), -1);
+        eallow_fp = max(wave_min_i32(eallow_fp), -1);
+        emax = wave_max_i32(emax);
     }
     const bool anybad = __builtin_amdgcn_ballot_w64(bad) != 0, anylbad = __builtin_amdgcn_ballot_w64(lbad) != 0;
-    if ((tid & 63) == 0) sh.wflag[tid >> 6] = (anybad ? 1 : 0) | (anylbad ? 2 : 0);
+    if ((tid & 63) == 0) sh.wflag[tid >> 6] = (anybad ? 1 : 0) | (anylbad ? 2 : 0) | (RX ? (__builtin_amdgcn_ballot_w64(bad_fp) != 0 ? 4 : 0) | (31 - eallow) << 8 | emax << 16 | (31 - eallow_fp) << 24 : 0);
     __syncthreads();   // raw table read by everyone, every wave's word in
     int f = 0;
 #pragma unroll
-    for (int w = 0; w < NT / 64; ++w) f |= sh.wflag[w];
+    for (int w = 0; w < NT / 64; ++w) {
+        const int fw = sh.wflag[w];
+        f |= fw & 7;
+        if constexpr (RX) {
+            eallow = min(eallow, 31 - ((fw >> 8) & 255));
+            emax = max(emax, (fw >> 16) & 255);
+            eallow_fp = min(eallow_fp, 31 - ((fw >> 24) & 255));
+        }
+    }
+    if (RX && emax > eallow) f |= 1;
+    if (RX && emax > eallow_fp) f |= 4;
     lut_ok = !NEEDLUT || !(f & 2);
     if constexpr (NEEDLUT) {
 #pragma unroll
@@ -191,13 +238,22 @@ __device__ __forceinline__ int stripe_setup(const GemmParams& p, StripeShared<EP
             if (i < 2050) sh.lut[i] = lv[q];
         }
     }
-    const int form = __builtin_amdgcn_readfirstlane(f == 0 ? FORM_INT : FORM_EXACT);
-    if (form == FORM_INT) {
+    const int form = __builtin_amdgcn_readfirstlane((f & 3) == 0 ? FORM_INT : RX && (f & 6) == 0 ? FORM_FP : FORM_EXACT);
+    if (form != FORM_EXACT) {
 #pragma unroll
         for (int q = 0; q < CPT; ++q) {
             const int j = tid + NT * q;
             if (j < ncols) {
                 const int4 c = cc[q];
+                if constexpr (RX) {
+                    if (form == FORM_FP) {
+                        sh.tab[j] = make_int4(c.x, c.y, c.z, int(128u * unsigned(c.w)));
+                        continue;
+                    }
+                    // s >= 1 where m != 0
+                    sh.tab[j] = make_int4(c.y ? int(unsigned(c.x) << (32 - c.y)) : 0, int(c.x ? 0x80000000u : 0u), c.z, int(128u * unsigned(c.w)));
+                    continue;
+                }
                 // C = 128 wsum m + 2^(s-1) + b 2^s (|C| < 2^63: |wsum| <= 128 Kp, s <= 31); GELU/GEGLU:
                 // the multiplier and C times 2^(32-s) (C's product wraps modulo 2^64; m = 0 when s = 0)
                 const i64 C = 128LL * i64(c.w) * i64(c.x) + (c.y ? (1LL << (c.y - 1)) : 0) + i64(c.z) * (1LL << c.y);
@@ -299,6 +355,28 @@ __device__ __forceinline__ StripeK3 stripe_tab3(const int4* tab, int j) {
 __device__ __forceinline__ int stripe_req_hi(int A, const StripeK3& k) {
     const i64 t = i64(A) * i64(k.m) + i64((u64(unsigned(k.hi)) << 32) | unsigned(k.lo));
     return int(unsigned(u64(t) >> 32));
+}
+
+// m << (byte V of e): the multiplier of an element of row V of a lane's four (e: their shifts, one a byte)
+template <int V>
+__device__ __forceinline__ int stripe_shl_row(int m, unsigned e) {
+    int r;
+    if constexpr (V == 0) asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_0 src1_sel:DWORD" : "=v"(r) : "v"(e), "v"(m));
+    if constexpr (V == 1) asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_1 src1_sel:DWORD" : "=v"(r) : "v"(e), "v"(m));
+    if constexpr (V == 2) asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_2 src1_sel:DWORD" : "=v"(r) : "v"(e), "v"(m));
+    if constexpr (V == 3) asm("v_lshlrev_b32_sdwa %0, %1, %2 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_3 src1_sel:DWORD" : "=v"(r) : "v"(e), "v"(m));
+    return r;
+}
+// the requantisation with row shifts: table entry k = {m 2^(32-s), 2^31, b, 128 wsum}
+template <int V>
+__device__ __forceinline__ int stripe_req_rx(int A, const int4& k, unsigned e) {
+    const i64 t = i64(A + k.w) * i64(stripe_shl_row<V>(k.x, e)) + i64((u64(unsigned(k.z)) << 32) | unsigned(k.y));
+    return int(unsigned(u64(t) >> 32));
+}
+
+// the same in double (FORM_FP): table entry k = {m, s, b, 128 wsum}, e the row's shift
+__device__ __forceinline__ int stripe_req_fp(int A, const int4& k, int e) {
+    return add_sat(cvt_sat(floor(fma(double(A + k.w), ldexp(double(k.x), e - k.y), 0.5))), k.z);
 }
 
 // RES: the PLAIN instantiation for calls with a residual (its own kernel, so that the residual
