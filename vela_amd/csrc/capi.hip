@@ -675,7 +675,11 @@ int hl2_impl(void* stream, const VgemmASrc* A, int Mp, int Mreal, const int8_t* 
     if (A->src == VGEMM_SRC_CONV32 && g_variant < 0 && p.C % 64 == 0) variant = 1;
     // int32 rows likewise (K % 4 == 0)
     if (A->src == VGEMM_SRC_X32 && g_variant < 0 && p.K % 4 == 0) variant = 1;
-    if (epi == VGEMM_EPI_QKV) variant = 0;   // whole heads per wave (the reference forces its 64 x 64 tile, src/gemm_hl.cu:358)
+    // whole heads per wave: 128 x 128 tiles, or 64 x 128 ones (int16 rows, int8 planes) while the larger leave
+    // CUs without a block (1024 x 640 x 1920, 120 tiles, 17.2 -> 12.3 us; 240 tiles 18.4 -> 17.4; from 512 tiles on
+    // the larger are ahead, 22.2 against 24.4). The reference forces its 64 x 64 tile (src/gemm_hl.cu:358).
+    if (epi == VGEMM_EPI_QKV)
+        variant = (A->src == VGEMM_SRC_I8 || A->src == VGEMM_SRC_I16) && (long long)cdiv(Mreal, TILES[0].BM) * cdiv(Nreal, TILES[0].BN) <= NCU ? 1 : 0;
     if (p.gnstat) {
         // statistics regions = the reference's tile; the block must hold whole regions (128 x 128
         // holds any of them, as does the halo kernel's 128 x 128)

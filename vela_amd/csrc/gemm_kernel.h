@@ -1587,8 +1587,10 @@ hipError_t launch_gemm_epi(int epi, const GemmParams& p, int batch, hipStream_t 
     case EPI_GELU: return VK_LAUNCH(EPI_GELU);
     case EPI_PARTIAL: return VK_LAUNCH(EPI_PARTIAL);
     case EPI_QKV:
-        // whole heads per wave: the 128 x 128 tiles only (the host selects variant 0)
-        if constexpr (std::is_same<T, TileD0>::value || std::is_same<T, TileV0>::value) return VK_LAUNCH(EPI_QKV);
+        // whole heads per wave: the 128 x 128 tiles, and 64 x 128 for int16 rows and int8 planes
+        if constexpr (std::is_same<T, TileD0>::value || std::is_same<T, TileV0>::value ||
+                      (std::is_same<T, TileD1>::value && (SRC == SRC_I8 || SRC == SRC_I16)))
+            return VK_LAUNCH(EPI_QKV);
         else return hipErrorInvalidValue;
     default: return hipErrorInvalidValue;
     }
