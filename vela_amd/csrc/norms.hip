@@ -707,7 +707,7 @@ static void tile_shape(int C, int rt_max, int& RT, int& NV) {
 
 // Tiles per block (whole rounds of its four waves): up to 32 rows, fewer while there would be less than four
 // blocks per CU (2048 rows of 640 as 64 blocks of 32 rows: LayerNorm 18.2 us; as 256 blocks of one tile a
-// wave LN_US), and for the GroupNorm apply at most 6 T + 1 rows, so that a block's rows span at most GN_SLOTS
+// wave 8.0 us), and for the GroupNorm apply at most 6 T + 1 rows, so that a block's rows span at most GN_SLOTS
 // samples (n consecutive rows span at most ceil((n - 1) / T) + 1 samples).
 static int tiles_per_block(long long M, int RT, long long row_cap) {
     const long long most = std::max<long long>(1, std::min<long long>(32, row_cap) / RT), spread = (M + RT - 1) / RT / 1024 / 4 * 4;
