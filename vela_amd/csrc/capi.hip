@@ -110,7 +110,7 @@ struct Tiles { int BM, BN; };
 // variant 3 (128 x 256, eight waves) exists for the DMA sources only; the register-staged sources
 // run it as variant 0
 constexpr int NVARIANT = 4;
-constexpr Tiles TILES[NVARIANT] = {{128, 128}, {64, 128}, {128, 64}, {128, 256}};
+constexpr Tiles TILES[NVARIANT + 1] = {{128, 128}, {64, 128}, {128, 64}, {128, 256}, {64, 320}};
 constexpr int NCU = 256;   // MI355X compute units
 
 int cdiv(long long a, long long b) { return int((a + b - 1) / b); }
@@ -266,6 +266,16 @@ int pick_variant_raw(int M, int N, int K) {
     if (K < 1024) return pick_variant(M, N, K);
     const long long tiles0 = (long long)cdiv(M, TILES[0].BM) * cdiv(N, TILES[0].BN);
     return tiles0 >= NCU ? 0 : 2;
+}
+
+// int32 rows on 64 x 320 tiles: no more padding columns than 128-wide tiles have, and the last round of blocks
+// (two per CU) at least three quarters full, since a round costs nearly the same with one block per CU (K = 1280, us,
+// 64 x 128 tiles first: 512 tiles 61.5 / 46.3, 448 tiles 58.0 / 44.7, 384 tiles 51.1 / 43.0, 256 tiles 32.2 / 37.0;
+// N = 1280: 512 tiles 54.9 / 46.3, 384 tiles 46.8 / 42.1; K = 320: 512 tiles 30 / 27, 256 tiles 17.4 / 22.4).
+bool x32_wide(int epi, const vk::GemmParams& p, int Kp) {
+    if (epi != VGEMM_EPI_PLAIN || p.gnstat || g_splitk > 1 || split_rule(p.Mreal, p.Nreal, Kp) != SPLIT_NONE) return false;
+    const long long tiles = (long long)cdiv(p.Mreal, 64) * cdiv(p.Nreal, 320), last = (tiles - 1) % (2 * NCU) + 1;
+    return cdiv(p.Nreal, 320) * 320 <= cdiv(p.Nreal, 128) * 128 && last >= 3 * NCU / 2;
 }
 
 int pick_splitk(int variant, int M, int N, int Kp) {
@@ -674,7 +684,7 @@ int hl2_impl(void* stream, const VgemmASrc* A, int Mp, int Mreal, const int8_t* 
     // rows in LDS and quantises them per fragment (C3 shape: 116 us, 218 us on the register-staged kernel)
     if (A->src == VGEMM_SRC_CONV32 && g_variant < 0 && p.C % 64 == 0) variant = 1;
     // int32 rows likewise (K % 4 == 0)
-    if (A->src == VGEMM_SRC_X32 && g_variant < 0 && p.K % 4 == 0) variant = 1;
+    if (A->src == VGEMM_SRC_X32 && g_variant < 0 && p.K % 4 == 0) variant = x32_wide(epi, p, Kp) ? vk::TILE_X32_WIDE : 1;
     // whole heads per wave: 128 x 128 tiles, or 64 x 128 ones (int16 rows, int8 planes) while the larger leave
     // CUs without a block (1024 x 640 x 1920, 120 tiles, 17.2 -> 12.3 us; 240 tiles 18.4 -> 17.4; from 512 tiles on
     // the larger are ahead, 22.2 against 24.4). The reference forces its 64 x 64 tile (src/gemm_hl.cu:358).

@@ -77,8 +77,8 @@ __global__ void __launch_bounds__(256, 2) conv_halo_kernel(const GemmParams p) {
         const int r = rbase + ms * 16 + (lane & 15);
         er[ms] = r < p.Mreal ? row_shift<SRC_CONV16>(p, r) : 0;
     }
-    TilePre pre{};
-    if constexpr (FUSED) pre = load_tile_pre<EPI, SRC_CONV16, BM, BN>(p, m0, n0);
+    TilePre<(BN + 255) / 256> pre{};
+    if constexpr (FUSED) pre = load_tile_pre<EPI, SRC_CONV16, BM, BN, 256>(p, m0, n0);
 
     const v4i rW = make_rsrc_words(p.w, p.w_bytes);
     const v4i rA = make_rsrc_words(p.a0, p.a0_bytes);

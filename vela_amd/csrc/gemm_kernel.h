@@ -54,6 +54,10 @@ typedef Tile<64, 128, 4, 1> TileD1;
 typedef Tile<128, 64, 4, 1> TileD2;
 // eight waves, 4 x 2: each A stripe feeds 256 columns (half the A traffic of 128-column tiles)
 typedef Tile<128, 256, 4, 2> TileD3;
+// int32 rows: each K step's rows are fetched, quantised and split once for 320 columns instead of once for every
+// 128 (what bounds the 64 x 128 tile: about 100 vector instructions a step beside 16 MFMAs). Two blocks of 78 KB
+// of LDS and at most 256 VGPRs a CU. 32768 x 1280 x 320 with the residual: 61.5 -> 46.3 us (252 MB at 5.4 TB/s).
+typedef Tile<64, 320, 4, 1> TileD4;
 
 // LDS layouts of the K-step tiles. A fragment load (ds_read_b128) has each group of 16 lanes read
 // one 16-byte chunk of 16 consecutive rows. Measured on gfx950 (a probe with SQ_LDS_BANK_CONFLICT):
@@ -410,21 +414,28 @@ __device__ __forceinline__ EpiFlags block_prologue(const GemmParams& p, int m0, 
 // first MFMA: the cst entry of table column tid and the shift of tile row tid are held in
 // registers (TilePre), and the GELU table arrives in LDS by DMA, raw, in the upper half of
 // sh.lut, and is expanded to (L[i], L[i+1] - L[i]) pairs here.
+template <int CPT>
 struct TilePre {
-    int4 c;
+    int4 c[CPT];
+    bool cok[CPT];
     int e;
-    bool cok, eok;
+    bool eok;
     int m0;
 };
 
-template <int EPI, int SRC, int BM, int BN>
-__device__ __forceinline__ TilePre load_tile_pre(const GemmParams& p, int m0, int n0) {
-    // one table row and one table column per thread (blocks have at least max(BM, BN) threads)
+template <int EPI, int SRC, int BM, int BN, int NT>
+__device__ __forceinline__ TilePre<(BN + NT - 1) / NT> load_tile_pre(const GemmParams& p, int m0, int n0) {
+    // one table row per thread and the table columns tid, tid + NT, ... (one, but for tiles wider than the block)
+    static_assert(NT >= BM, "one table row per thread");
+    constexpr int CPT = (BN + NT - 1) / NT;
     const int tid = threadIdx.x;
-    TilePre t;
-    const int n = n0 + wrow_of_lds<EPI, BN>(tid < BN ? tid : 0);
-    t.cok = tid < BN && n < p.Nreal;
-    t.c = t.cok ? p.cst[n] : make_int4(0, 0, 0, 0);
+    TilePre<CPT> t;
+#pragma unroll
+    for (int c = 0; c < CPT; ++c) {
+        const int j = tid + NT * c, n = n0 + wrow_of_lds<EPI, BN>(j < BN ? j : 0);
+        t.cok[c] = j < BN && n < p.Nreal;
+        t.c[c] = t.cok[c] ? p.cst[n] : make_int4(0, 0, 0, 0);
+    }
     const int r = m0 + tid;
     t.eok = tid < BM && r < p.Mreal;
     t.e = t.eok ? (row_shift<SRC>(p, r)) : 0;
@@ -436,9 +447,9 @@ __device__ __forceinline__ TilePre load_tile_pre(const GemmParams& p, int m0, in
 constexpr unsigned LUT_RAW_OFF = 8192;
 
 template <int EPI, int SRC, int BM, int BN, int NT, class S>
-__device__ __forceinline__ EpiFlags epi_setup(const GemmParams& p, const TilePre& t, int L2048, S& sh) {
+__device__ __forceinline__ EpiFlags epi_setup(const GemmParams& p, const TilePre<(BN + NT - 1) / NT>& t, int L2048, S& sh) {
     constexpr bool NEEDLUT = EPI == EPI_GEGLU || EPI == EPI_GELU;
-    static_assert(NT >= BM && NT >= BN, "one table row and column per thread");
+    constexpr int CPT = (BN + NT - 1) / NT;
     const int tid = threadIdx.x;
     // ---- phase 1: everything that reads LDS or needs no LDS (the raw table is still in place)
     constexpr int LPT = NEEDLUT ? (2050 + NT - 1) / NT : 1;   // table entries per thread
@@ -459,9 +470,10 @@ __device__ __forceinline__ EpiFlags epi_setup(const GemmParams& p, const TilePre
             lv[q] = v;
         }
     }
-    double ms = 0.0, wmv = 0.0;
-    const int bb = t.cok ? t.c.z : 0;
-    if (t.cok) setup_column(p, t.c, ms, wmv, sp);
+    double ms[CPT] = {}, wmv[CPT] = {};
+#pragma unroll
+    for (int c = 0; c < CPT; ++c)
+        if (t.cok[c]) setup_column(p, t.c[c], ms[c], wmv[c], sp);
     if (t.eok) { sp.emn = t.e; sp.emx = t.e; }
     setup_publish(sh, sp);
     if constexpr (EPI == EPI_PLAIN_GN) gn_clear(p, t.m0, sh);
@@ -469,10 +481,14 @@ __device__ __forceinline__ EpiFlags epi_setup(const GemmParams& p, const TilePre
     // ---- phase 2: the block's forms, the column tables (with the e == 0 FMA constant: wm + 1/2, and
     // + b when folded, exact as above) and the expanded GELU table
     const EpiFlags f = setup_flags<NEEDLUT, NT / 64>(sh);
-    if (tid < BN) {
-        sh.ms[tid] = ms;
-        sh.wm[tid] = f.ezero ? (wmv + 0.5) + (f.fold ? double(bb) : 0.0) : wmv;
-        sh.b[tid] = bb;
+#pragma unroll
+    for (int c = 0; c < CPT; ++c) {
+        const int j = tid + NT * c, bb = t.c[c].z;   // zero where there is no column
+        if (j < BN) {
+            sh.ms[j] = ms[c];
+            sh.wm[j] = f.ezero ? (wmv[c] + 0.5) + (f.fold ? double(bb) : 0.0) : wmv[c];
+            sh.b[j] = bb;
+        }
     }
     if constexpr (NEEDLUT) {
 #pragma unroll
@@ -986,8 +1002,8 @@ __global__ void __launch_bounds__(T::NT, (dma_waves_per_simd<T, EPI>())) gemm_dm
         const int r = rbase + ms * 16 + (lane & 15);
         er[ms] = (r < p.Mreal && (FUSED || D::RAW32 || SRC == SRC_CONV16)) ? row_shift<SRC>(p, r) : 0;
     }
-    TilePre pre{};
-    if constexpr (FUSED) pre = load_tile_pre<EPI, SRC, BM, BN>(p, m0, n0);
+    TilePre<(BN + T::NT - 1) / T::NT> pre{};
+    if constexpr (FUSED) pre = load_tile_pre<EPI, SRC, BM, BN, T::NT>(p, m0, n0);
     const int L2048 = D::NEEDLUT ? p.Lphi[2048] : 0;
     if constexpr (D::NEEDLUT) {
         // GELU table entries 0..2047 -> LDS (raw), 8 KB: eight 1 KB DMA instructions per block
@@ -1597,7 +1613,7 @@ hipError_t launch_gemm_epi(int epi, const GemmParams& p, int batch, hipStream_t 
 #undef VK_LAUNCH
 }
 
-// variant -> tile: 0 = 128x128, 1 = 64x128, 2 = 128x64 (rows x columns)
+// variant -> tile: 0 = 128x128, 1 = 64x128, 2 = 128x64 (rows x columns); int32 rows also 64x320
 template <int SRC>
 hipError_t launch_gemm_src(int variant, int epi, const GemmParams& p, int batch, hipStream_t st) {
     constexpr bool DMA = SRC == SRC_I8 || SRC == SRC_I16 || SRC == SRC_CONV16;
@@ -1613,8 +1629,10 @@ hipError_t launch_gemm_src(int variant, int epi, const GemmParams& p, int batch,
         // kernel (raw int32 rows in LDS)
         if constexpr (SRC == SRC_CONV32)
             if (variant == 1 && (p.C & 63) == 0) return launch_gemm_epi<SRC, TileD1, true>(epi, p, batch, st);
-        if constexpr (SRC == SRC_X32)
+        if constexpr (SRC == SRC_X32) {
+            if (variant == TILE_X32_WIDE) return epi == EPI_PLAIN ? launch_dma_t<SRC, EPI_PLAIN, TileD4>(p, batch, st) : hipErrorInvalidValue;
             if (variant == 1 && (p.K & 3) == 0) return launch_gemm_epi<SRC, TileD1, true>(epi, p, batch, st);
+        }
         switch (variant) {
         case 1: return launch_gemm_epi<SRC, TileV1, false>(epi, p, batch, st);
         case 2: return launch_gemm_epi<SRC, TileV2, false>(epi, p, batch, st);

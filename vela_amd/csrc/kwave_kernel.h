@@ -61,7 +61,7 @@ __global__ void __launch_bounds__(256, SRC == SRC_I8 ? 2 : 1) kwave_kernel(const
         const int r = m0 + ms * 16 + fr;
         er4[ms] = r < p.Mreal ? row_shift<SRC>(p, r) : 0;
     }
-    const TilePre pre = load_tile_pre<EPI, SRC, 64, 64>(p, m0, n0);
+    const TilePre<1> pre = load_tile_pre<EPI, SRC, 64, 64, 256>(p, m0, n0);
     const int L2048 = NEEDLUT ? p.Lphi[2048] : 0;
     if constexpr (NEEDLUT) {
         // GELU table entries 0..2047 -> LDS (raw), 8 KB: two 1 KB DMA instructions per wave

@@ -33,6 +33,8 @@ constexpr unsigned OOB = 0x80000000u;
 // Third descriptor word of a raw (untyped) buffer resource on gfx9-family GPUs.
 constexpr int RSRC_WORD3 = 0x00020000;
 
+constexpr int TILE_X32_WIDE = 4;   // tile variant of int32 rows, 64 x 320, beyond the ones that can be forced
+
 struct GemmParams {
     // A operand
     const void* a0;            // hi plane / q16 / x / img / img16
