@@ -40,7 +40,8 @@ def ptr(t) -> int | None:
 
 def stream_ptr(stream=None) -> int | None:
     if stream is None:
-        stream = torch.cuda.current_stream()
+        # the raw handle, without building a Stream object for each launch
+        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()) or None
     if isinstance(stream, int):
         return stream or None
     return stream.cuda_stream or None
