@@ -13,6 +13,7 @@
 #include "../../include/vgemm.h"
 #include "vk_common.h"
 #include "attn.h"
+#include "dispatch_rules.h"
 
 namespace vk {
 hipError_t launch_gemm_i8(int variant, int epi, const GemmParams& p, int batch, hipStream_t st);
@@ -111,9 +112,8 @@ struct Tiles { int BM, BN; };
 // run it as variant 0
 constexpr int NVARIANT = 4;
 constexpr Tiles TILES[NVARIANT + 1] = {{128, 128}, {64, 128}, {128, 64}, {128, 256}, {64, 320}};
-constexpr int NCU = 256;   // MI355X compute units
-
-int cdiv(long long a, long long b) { return int((a + b - 1) / b); }
+using vk::cdiv;
+using vk::NCU;
 
 // Variant 4 forces the row-stationary kernel (stripe_kernel.h) where it applies: int16 rows or int8
 // planes, epilogue PLAIN (with or without a residual) / GEGLU / GELU, Kp <= 320, output columns in
@@ -268,14 +268,9 @@ int pick_variant_raw(int M, int N, int K) {
     return tiles0 >= NCU ? 0 : 2;
 }
 
-// int32 rows on 64 x 320 tiles: no more padding columns than 128-wide tiles have, and the last round of blocks
-// (two per CU) at least three quarters full, since a round costs nearly the same with one block per CU (K = 1280, us,
-// 64 x 128 tiles first: 512 tiles 61.5 / 46.3, 448 tiles 58.0 / 44.7, 384 tiles 51.1 / 43.0, 256 tiles 32.2 / 37.0;
-// N = 1280: 512 tiles 54.9 / 46.3, 384 tiles 46.8 / 42.1; K = 320: 512 tiles 30 / 27, 256 tiles 17.4 / 22.4).
 bool x32_wide(int epi, const vk::GemmParams& p, int Kp) {
     if (epi != VGEMM_EPI_PLAIN || p.gnstat || g_splitk > 1 || split_rule(p.Mreal, p.Nreal, Kp) != SPLIT_NONE) return false;
-    const long long tiles = (long long)cdiv(p.Mreal, 64) * cdiv(p.Nreal, 320), last = (tiles - 1) % (2 * NCU) + 1;
-    return cdiv(p.Nreal, 320) * 320 <= cdiv(p.Nreal, 128) * 128 && last >= 3 * NCU / 2;
+    return vk::x32_wide_tiles(p.Mreal, p.Nreal, Kp);
 }
 
 int pick_splitk(int variant, int M, int N, int Kp) {
