@@ -10,6 +10,7 @@ ROOT = Path(__file__).resolve().parent.parent
 EXPORTS = """
 #include "dispatch_rules.h"
 extern "C" int x32_wide_tiles(int M, int N, int Kp) { return vk::x32_wide_tiles(M, N, Kp); }
+extern "C" int stripe_shift_rows(int epi, int M, int N, int Kp) { return vk::stripe_shift_rows(vk::ShiftEpi(epi), M, N, Kp); }
 """
 
 
@@ -40,3 +41,28 @@ def rules(tmp_path_factory):
 ])
 def test_int32_rows_on_wide_tiles(rules, M, N, K, wide):
     assert bool(rules.x32_wide_tiles(M, N, K)) == wide
+
+
+@pytest.mark.parametrize("epi,M,N,K,row_stationary", [
+    (1, 32768, 2560, 320, True), (1, 4096, 2560, 320, True), (1, 3520, 2560, 320, True), (1, 6592, 2560, 320, True), (0, 32768, 320, 320, True),
+    (0, 16384, 1280, 320, True), (0, 3136, 2560, 320, True), (0, 7040, 1280, 320, True), (0, 12352, 640, 320, True), (0, 20544, 320, 160, True),
+    (0, 64000, 320, 320, True), (1, 65536, 256, 192, True),
+    (0, 61568, 64, 320, True), (1, 38400, 640, 320, True), (1, 76083, 640, 304, True), (1, 30374, 640, 320, True), (0, 12867, 2104, 128, True), (2, 69866, 320, 304, True),
+    (2, 7040, 1280, 320, True), (2, 9932, 2560, 96, True), (2, 13120, 1280, 64, True),
+    # slower there (tile kernels / row-stationary, us): one chunk a block, grids just past a whole number of rounds
+    (0, 61568, 72, 320, False),      # 16.5 / 20.6
+    (1, 61568, 128, 320, False),     # 21.0 / 23.7
+    (0, 14080, 640, 320, False),     # 19.8 / 20.4, 22.4 in double
+    (0, 16640, 640, 320, False),     # 21.9 / 23.2, 26.1 in double
+    (1, 23488, 328, 320, False),     # 20.5 / 22.0
+    (0, 24576, 512, 320, False),     # 23.4 / 25.3 in double
+    (1, 2944, 2568, 320, False),     # 16.1 / 17.1 in double
+    (1, 4713, 2560, 320, False),     # 24.7 / 25.2, 27.8 in double
+    # five K steps whatever Kp is
+    (1, 61568, 72, 64, False), (0, 24576, 512, 64, False), (1, 3136, 2560, 64, False), (1, 10844, 2560, 96, False), (2, 3136, 2560, 64, False),
+    # few rows, few tiles
+    (0, 16384, 320, 320, False), (1, 1000, 8000, 320, False), (1, 1400, 2560, 320, False),
+])
+def test_rows_with_shifts(rules, epi, M, N, K, row_stationary):
+    """epi 0 PLAIN, 1 GEGLU, 2 GELU."""
+    assert bool(rules.stripe_shift_rows(epi, M, N, K)) == row_stationary

@@ -47,3 +47,10 @@ def test_edges(epi, M, N, K):
 def test_automatic_route(e_max):
     """3100 x 320 x 2560: 980 tiles of 64x128, the row-stationary kernels with and without shifts."""
     Case(vg.SRC_I8, 3100, 2560, 320, epi=vg.EPI_GEGLU, seed=5 + e_max, rowmax=True, s_range=(23, 26), e_max=e_max).check(what=f"auto e {e_max}")
+
+
+@pytest.mark.parametrize("epi,M,N,K", [(vg.EPI_GEGLU, 3520, 2560, 320), (vg.EPI_GEGLU, 6592, 2560, 304), (vg.EPI_PLAIN, 20544, 320, 160), (vg.EPI_GELU, 7040, 1280, 320),
+                                       (vg.EPI_GELU, 8320, 1280, 64)])
+def test_automatic_route_by_ranges(epi, M, N, K):
+    """Grids of one round and of more that the rule on a block's chunks sends to the row-stationary kernel."""
+    Case(vg.SRC_I8, M, N, K, epi=epi, seed=M, rowmax=True, s_range=(23, 26), e_max=6).check(what=f"auto {epi} {M}x{K}x{N}")

@@ -133,8 +133,7 @@ constexpr int VARIANT_STRIPE16 = 6;
 // fragment for twice the rows (16-row waves double the LDS reads: 32768 x 320 x 2560 PLAIN 78.9 ->
 // 83.8 us on stripe16).
 bool stripe16_auto(int epi) { return epi == VGEMM_EPI_GEGLU || epi == VGEMM_EPI_GELU; }
-constexpr int STRIPE_BM = 128, STRIPE_CH = 64;
-constexpr int STRIPE_NCOLS = 1280;   // W rows per block, at most
+using vk::STRIPE_BM;
 
 bool stripe_applies(int src, int epi, const vk::GemmParams& p) {
     if (src != VGEMM_SRC_I16 && src != VGEMM_SRC_I8) return false;
@@ -170,21 +169,8 @@ bool kwave_auto(const vk::GemmParams& p) {
            (long long)cdiv(p.Mreal, 64) * cdiv(p.Nreal, 64) <= NCU;
 }
 
-// Blocks = row stripes x column ranges: as few column ranges as the table allows, raised until
-// there are two blocks per CU. Returns the column ranges and the chunks of each.
-void stripe_ranges(const vk::GemmParams& p, int& cs, int& kper) {
-    const int nch = cdiv(p.Nreal, STRIPE_CH);
-    const int mt = cdiv(p.Mreal, STRIPE_BM);
-    cs = std::max(cdiv(nch, STRIPE_NCOLS / STRIPE_CH), std::min(nch, cdiv(2 * NCU, mt)));
-    kper = cdiv(nch, cs);
-    cs = cdiv(nch, kper);
-}
-
-// Automatic use. Calls with per-row shifts run the sixteen-row kernel's form for them, PLAIN too (32768 x 320
-// with row shifts: x 2560 GEGLU 118.3 -> 66.4 us, x 320 PLAIN 20.4 -> 16.9, 16384 x 320 x 1280 GELU 39.7 ->
-// 25.4, against the tile kernels), by the last rule below alone (3096 x 320 x 2560, 980 tiles, 18.3 -> 16.9;
-// below it the tile kernels stay ahead: 16384 x 320 x 320, 768 tiles, 12.3 against 13.4, 1400 x 320 x 2560,
-// 440 tiles, 10.9 against 14.7) and not with a residual, which that kernel does not add. Without shifts:
+// Automatic use. Calls with per-row shifts: vk::stripe_shift_rows, and not with a residual, which the sixteen-row
+// kernel (the only one with a form for shifts) does not add. Without shifts:
 //  * many rows (a block keeps its rows in registers and streams its columns, so the kernels need a
 //    few hundred row stripes to fill the GPU); residual calls qualify, the kernel loading a batch's
 //    residuals ahead of its arithmetic (UNet 32768 x 320 x 320 residual layers: 23.1 us against
@@ -200,19 +186,19 @@ void stripe_ranges(const vk::GemmParams& p, int& cs, int& kper) {
 //    29.4 -> 21.1, 960 tiles 4-16 % faster; at 640 and 768 tiles the tile kernels stay ahead,
 //    4096 x 320 x 1280 PLAIN 11.2 against 12.1 us).
 bool stripe_auto(int epi, const vk::GemmParams& p) {
-    if (p.e) return !p.R && p.Mreal >= 1024 && (long long)cdiv(p.Mreal, 64) * cdiv(p.Nreal, 128) >= 15LL * NCU / 4;
+    if (p.e) {
+        const vk::ShiftEpi se = epi == VGEMM_EPI_GEGLU ? vk::SHIFT_GEGLU : epi == VGEMM_EPI_GELU ? vk::SHIFT_GELU : vk::SHIFT_PLAIN;
+        return !p.R && vk::stripe_shift_rows(se, p.Mreal, p.Nreal, p.Kp);
+    }
     if (cdiv(p.Mreal, STRIPE_BM) >= 2 * NCU / 4 && p.Mreal >= 16384) return true;
     if (p.Mreal >= 1024 && (long long)cdiv(p.Mreal, 64) * cdiv(p.Nreal, 128) >= 15LL * NCU / 4) return true;
-    int cs, kper;
-    stripe_ranges(p, cs, kper);
-    return (long long)cdiv(p.Mreal, STRIPE_BM) * cs <= NCU;
+    return (long long)cdiv(p.Mreal, STRIPE_BM) * vk::stripe_ranges(p.Mreal, p.Nreal).cs <= NCU;
 }
 
 constexpr int STRIPE_PRIO_PCT = 55;
 void stripe_grid(vk::GemmParams& p) {
     const int mt = cdiv(p.Mreal, STRIPE_BM);
-    int cs, kper;
-    stripe_ranges(p, cs, kper);
+    const auto [cs, kper] = vk::stripe_ranges(p.Mreal, p.Nreal);
     p.mtiles = mt;
     p.ntiles = cs;
     p.kper = kper;
