@@ -11,6 +11,9 @@ EXPORTS = """
 #include "dispatch_rules.h"
 extern "C" int x32_wide_tiles(int M, int N, int Kp) { return vk::x32_wide_tiles(M, N, Kp); }
 extern "C" int stripe_shift_rows(int epi, int M, int N, int Kp) { return vk::stripe_shift_rows(vk::ShiftEpi(epi), M, N, Kp); }
+extern "C" int norm_tiles(int gn, long long M, int RT, long long row_cap) {
+    return vk::norm_tiles_per_block(M, RT, row_cap, gn ? vk::GN_APPLY_COST : vk::LNORM_COST);
+}
 """
 
 
@@ -66,3 +69,24 @@ def test_int32_rows_on_wide_tiles(rules, M, N, K, wide):
 def test_rows_with_shifts(rules, epi, M, N, K, row_stationary):
     """epi 0 PLAIN, 1 GEGLU, 2 GELU."""
     assert bool(rules.stripe_shift_rows(epi, M, N, K)) == row_stationary
+
+
+@pytest.mark.parametrize("gn,M,RT,tiles", [
+    # few rows: one tile a wave
+    (0, 64, 1, 4), (0, 2048, 2, 4), (0, 1024, 4, 4), (1, 256, 1, 4), (1, 2048, 2, 4), (1, 4096, 4, 4),
+    # whole numbers of blocks a CU (12 tiles a block, 1360 blocks, 77.7 -> 91.8 us of GroupNorm + SiLU, 16320 x 1920)
+    (0, 16320, 1, 16), (1, 16320, 1, 32), (1, 16320, 4, 8), (1, 23108, 4, 8), (1, 32720, 4, 8), (0, 32720, 2, 16), (1, 13716, 2, 16),
+    # between them, fewer rows a block
+    (1, 11528, 4, 4), (0, 9688, 1, 8), (1, 9688, 1, 20), (1, 18000, 1, 12), (1, 13716, 1, 28), (1, 131072, 4, 8),
+])
+def test_norm_tiles(rules, gn, M, RT, tiles):
+    assert rules.norm_tiles(gn, ctypes.c_longlong(M), RT, ctypes.c_longlong(1 << 20)) == tiles
+
+
+@pytest.mark.parametrize("T", [1, 2, 3, 5, 7, 100])
+@pytest.mark.parametrize("RT", [1, 2, 4, 8])
+def test_norm_tiles_span(rules, T, RT):
+    """A block of the GroupNorm apply spans at most eight samples, so at most 6 T + 1 rows (or one tile)."""
+    for M in (T, 1000 * T + 1, 40000 * T):
+        t = rules.norm_tiles(1, ctypes.c_longlong(M), RT, ctypes.c_longlong(6 * T + 1))
+        assert 1 <= t and (t == 1 or t * RT <= min(32, 6 * T + 1))

@@ -232,3 +232,51 @@ def test_gn_apply_row_silu_tables(gpu, table):
     assert_equal(to_np(pm).view(np.uint32), pmw, f"{table} pm")
     for got, w, n in zip((hi, lo, e), oracle.gn_apply_row(x, B, T, C, groups, st, g, beta, Lsig=L, Kp=Kp), ("hi", "lo", "e")):
         assert_equal(to_np(got), w, f"{table} {n}")
+
+
+@pytest.mark.parametrize("M,C", [(9687, 512), (16321, 1920), (32717, 320), (32721, 640)])
+def test_lnorm_many_tiles(gpu, M, C):
+    """Blocks whose waves take several tiles each, the last block short: 8 and 16 tiles of one row,
+    8 of four, 16 of two."""
+    r = np.random.default_rng(M + C)
+    x = make_x(r, M, C, 1)
+    x[:: 97] //= 50000                                     # rows of other sizes
+    g, beta = r.integers(30000, 90000, C).astype(np.int32), r.integers(-20000, 20000, C).astype(np.int32)
+    den, Kp = 100000, (C + 15) // 16 * 16
+    X = dev(x)
+    hi, lo = (torch.full((M, Kp), 0x5a, dtype=torch.int8, device="cuda") for _ in range(2))
+    e = torch.full((M,), 0x5a5a5a5a, dtype=torch.int32, device="cuda")
+    vn.k_lnorm_q(X, M, C, dev(g), dev(beta), den, hi, lo, e, Kp)
+    Y = torch.full((M, C), 0x5a5a5a5a, dtype=torch.int32, device="cuda")
+    vn.k_lnorm(X, M, C, dev(g.astype(np.int64)), dev(beta.astype(np.int64)), den, Y)
+    torch.cuda.synchronize()
+    for got, w, n in zip((hi, lo, e), oracle.lnorm_q(x, M, C, g, beta, den, Kp), ("hi", "lo", "e")):
+        assert_equal(to_np(got), w, f"lnorm_q {M}x{C} {n}")
+    assert_equal(to_np(Y), oracle.lnorm(x, M, C, g.astype(np.int64), beta.astype(np.int64), den), f"lnorm {M}x{C}")
+
+
+@pytest.mark.parametrize("B,T,C", [(4, 4079, 320), (3, 3229, 512), (1400, 7, 512), (800, 17, 320), (2, 6857, 640)])
+def test_gn_apply_row_many_tiles(gpu, B, T, C):
+    """Blocks whose waves take several tiles each, spanning one, two, and up to five samples."""
+    r = np.random.default_rng(B * T + C)
+    groups, M, Kp = 32, B * T, (C + 15) // 16 * 16
+    x = make_x(r, M, C, 1)
+    g, beta = r.integers(30000, 90000, C).astype(np.int32), r.integers(-20000, 20000, C).astype(np.int32)
+    L = (np.arange(2049) * 32).astype(np.int32)
+    st = oracle.gn_records(B * groups)
+    st["mean"] = r.integers(-500000, 500001, B * groups)
+    st["e"] = 0
+    st["sd"] = 65536 + r.integers(0, 100000000, B * groups)
+    X, G, Bt, Ld, S = dev(x), dev(g), dev(beta), dev(L), records_dev(st)
+    Y = torch.full((M, C), 0x5a5a5a5a, dtype=torch.int32, device="cuda")
+    pm = torch.full((M,), 0x5a5a5a5a, dtype=torch.int32, device="cuda")
+    vn.k_gn_apply_row(X, B, T, C, groups, S, G, Bt, Ld, Y, pm, None, None, None, 0)
+    hi, lo = (torch.full((M, Kp), 0x5a, dtype=torch.int8, device="cuda") for _ in range(2))
+    e = torch.full((M,), 0x5a5a5a5a, dtype=torch.int32, device="cuda")
+    vn.k_gn_apply_row(X, B, T, C, groups, S, G, Bt, Ld, None, None, hi, lo, e, Kp)
+    torch.cuda.synchronize()
+    Yw, pmw = oracle.gn_apply_row(x, B, T, C, groups, st, g, beta, Lsig=L)
+    assert_equal(to_np(Y), Yw, f"{B}x{T}x{C} Y")
+    assert_equal(to_np(pm).view(np.uint32), pmw, f"{B}x{T}x{C} pm")
+    for got, w, n in zip((hi, lo, e), oracle.gn_apply_row(x, B, T, C, groups, st, g, beta, Lsig=L, Kp=Kp), ("hi", "lo", "e")):
+        assert_equal(to_np(got), w, f"{B}x{T}x{C} {n}")

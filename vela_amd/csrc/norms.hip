@@ -24,6 +24,7 @@
 #include <algorithm>
 #include <climits>
 
+#include "dispatch_rules.h"
 #include "vk_common.h"
 
 namespace vk {
@@ -705,20 +706,13 @@ static void tile_shape(int C, int rt_max, int& RT, int& NV) {
     }
 }
 
-// Tiles per block (whole rounds of its four waves): up to 32 rows, fewer while there would be less than four
-// blocks per CU (2048 rows of 640 as 64 blocks of 32 rows: LayerNorm 18.2 us; as 256 blocks of one tile a
-// wave 8.0 us), and for the GroupNorm apply at most 6 T + 1 rows, so that a block's rows span at most GN_SLOTS
-// samples (n consecutive rows span at most ceil((n - 1) / T) + 1 samples).
-static int tiles_per_block(long long M, int RT, long long row_cap) {
-    const long long most = std::max<long long>(1, std::min<long long>(32, row_cap) / RT), spread = (M + RT - 1) / RT / 1024 / 4 * 4;
-    return int(std::min(most, std::max<long long>(4, spread)));
-}
-
 hipError_t launch_gn_apply_row(hipStream_t st, const int32_t* X, int M, int T, int C, int groups, const GnStat* gs, const int32_t* g, const int32_t* beta,
                                const int32_t* Lsig, int32_t* Y, uint32_t* pm, int8_t* hi, int8_t* lo, int32_t* e, int Kp) {
     int RT, NV;
     tile_shape(C, int(std::min<long long>(8, 6LL * T + 1)), RT, NV);
-    const int tpb = tiles_per_block(M, RT, 6LL * T + 1);
+    // at most 6 T + 1 rows a block, so that they span at most GN_SLOTS samples (n consecutive rows span at most
+    // ceil((n - 1) / T) + 1)
+    const int tpb = norm_tiles_per_block(M, RT, 6LL * T + 1, GN_APPLY_COST);
     const GnApplyArgs a{X, M, T, C, groups, RT, tpb, gs, g, beta, Y, pm, hi, lo, e, Kp};
     const dim3 grid(nblocks(nblocks(M, RT), tpb));
     const size_t lds = sizeof(NormK) * GN_SLOTS * GN_MAXG + 2 * sizeof(int32_t) * C + (Lsig ? sizeof(int32_t) * LUT_N : 0);
@@ -742,7 +736,7 @@ hipError_t launch_lnorm(hipStream_t st, bool q, const int32_t* X, int M, int C, 
     for (int ex = 0; ex < 13; ++ex) eps.v[ex] = ((1LL << (32 - 2 * ex)) + den / 2) / den;   // positive operands: the quotient is the floor
     int RT, NV;
     tile_shape(C, 8, RT, NV);
-    const int tpb = tiles_per_block(M, RT, 32);
+    const int tpb = norm_tiles_per_block(M, RT, 32, LNORM_COST);
     const dim3 grid(nblocks(nblocks(M, RT), tpb));
     const size_t lds = q ? 2 * sizeof(int32_t) * C : 0;
 #define VK_LNORM(N, QQ) hipLaunchKernelGGL((lnorm_kernel<N, QQ>), grid, dim3(256), lds, st, X, M, C, RT, tpb, g, beta, eps, Y, hi, lo, e, Kp)
