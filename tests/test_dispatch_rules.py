@@ -14,6 +14,7 @@ extern "C" int stripe_shift_rows(int epi, int M, int N, int Kp) { return vk::str
 extern "C" int norm_tiles(int gn, long long M, int RT, long long row_cap) {
     return vk::norm_tiles_per_block(M, RT, row_cap, gn ? vk::GN_APPLY_COST : vk::LNORM_COST);
 }
+extern "C" int attn_form(int Tkp) { const vk::AttnForm f = vk::attn_form(Tkp); return f.multi ? 0 : 10 * f.waves + f.tiles; }
 """
 
 
@@ -90,3 +91,14 @@ def test_norm_tiles_span(rules, T, RT):
     for M in (T, 1000 * T + 1, 40000 * T):
         t = rules.norm_tiles(1, ctypes.c_longlong(M), RT, ctypes.c_longlong(6 * T + 1))
         assert 1 <= t and (t == 1 or t * RT <= min(32, 6 * T + 1))
+
+
+@pytest.mark.parametrize("Tkp", range(64, 1280, 64))
+def test_attention_form(rules, Tkp):
+    """The kept forms hold every tile of the keys, and up to 256 keys no more than the next power of two of them."""
+    f = rules.attn_form(Tkp)
+    assert (f == 0) == (Tkp > 1024)
+    if f:
+        waves, tiles = f // 10, f % 10
+        assert waves * tiles * 64 >= Tkp
+        assert waves * tiles * 64 < 2 * Tkp

@@ -102,3 +102,11 @@ def test_dominant_key(gpu):
     """One key takes a row's whole probability (sum of E = 2^30, r = 2^32, P = 32768 before the clamp)."""
     for Tk in (3, 200, 1100):
         check(1, 1, 33, Tk, False, scale=600000)
+
+
+@pytest.mark.parametrize("Tk", [1, 3, 20, 63, 64])
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("kw", [dict(), dict(table=RISING), dict(table=SMALL), dict(scale=20000000)])
+def test_one_tile(gpu, Tk, causal, kw):
+    """Keys of one tile, in the integer arithmetic and in the general one."""
+    check(2, 3, 70, Tk, causal, **kw)

@@ -38,6 +38,7 @@
 #include <climits>
 
 #include "attn.h"
+#include "dispatch_rules.h"
 
 namespace vk {
 
@@ -813,20 +814,17 @@ __global__ void __launch_bounds__(256) quant_v_write_kernel(const int32_t* __res
 
 // ---------------------------------------------------------------- launchers
 
-// Four waves a block. Up to 256 keys (Tkp) a wave holds all of its queries' scores, up to 1024 two or four
-// waves split the keys (80 groups of 1024 x 1024: 119 us, against 187 when every pass recomputes the
-// scores); beyond, the recomputing form, as eight or sixteen waves to a row's scores leave 128 registers
-// each, where they spill (4096 x 4096, 40 groups: 2350 us so, 1420 recomputed; 2795 in the form that
-// recomputed them in double for every wave). The register limits are what measured best of 2, 3 and 4 waves
-// per SIMD.
+// Four waves a block, in the form that attn_form gives. The register limits are what measured best of 2, 3 and 4
+// waves per SIMD.
 hipError_t launch_attention(hipStream_t st, const AttnArgs& a, int G) {
-    const bool multi = a.Tkp > 1024;
-    const int KW = multi || a.Tkp <= 256 ? 1 : a.Tkp <= 512 ? 2 : 4, QW = 4 / KW;
+    const AttnForm f = attn_form(a.Tkp);
+    const int KW = f.waves, QW = 4 / KW;
     const int qblocks = (a.Tq + 16 * QW - 1) / (16 * QW);
-    const unsigned lds = attn_layout(4, QW, KW, multi ? std::min(a.Tkp, KEY_RANGE) : a.Tkp).bytes;
+    const unsigned lds = attn_layout(4, QW, KW, f.multi ? std::min(a.Tkp, KEY_RANGE) : a.Tkp).bytes;
     const dim3 grid(unsigned(qblocks * G)), blk(256);
-    if (multi) hipLaunchKernelGGL((attn_kernel<1, true, 256, 2>), grid, blk, lds, st, a, QW, KW, qblocks);
-    else if (a.Tkp <= 128) hipLaunchKernelGGL((attn_kernel<2, false, 256, 4>), grid, blk, lds, st, a, QW, KW, qblocks);
+    if (f.multi) hipLaunchKernelGGL((attn_kernel<1, true, 256, 2>), grid, blk, lds, st, a, QW, KW, qblocks);
+    else if (f.tiles == 1) hipLaunchKernelGGL((attn_kernel<1, false, 256, 4>), grid, blk, lds, st, a, QW, KW, qblocks);
+    else if (f.tiles == 2) hipLaunchKernelGGL((attn_kernel<2, false, 256, 4>), grid, blk, lds, st, a, QW, KW, qblocks);
     else hipLaunchKernelGGL((attn_kernel<4, false, 256, 3>), grid, blk, lds, st, a, QW, KW, qblocks);
     return hipGetLastError();
 }

@@ -93,4 +93,18 @@ inline int norm_tiles_per_block(long long M, int RT, long long row_cap, NormCost
     return best;
 }
 
+// The attention's form for Tkp padded keys: the waves that split a row's keys and the 64-key tiles of scores that each
+// holds, or (multi) one wave that recomputes the scores in each pass. Up to 256 keys a wave holds all of its queries'
+// scores, with a form of one tile for up to 64 keys (with two, 10 groups of 1024 x 20 in the general arithmetic 13.4 us
+// in place of 11.3, 160 groups of 1024 x 64 in the integer one 39.6 in place of 28.7), up to 1024 two or four waves split
+// the keys (80 groups of 1024 x 1024: 119 us, against 187 when every pass recomputes the scores); beyond, the recomputing
+// form, as eight or sixteen waves to a row's scores leave 128 registers each, where they spill (4096 x 4096, 40 groups:
+// 2350 us so, 1420 recomputed; 2795 in the form that recomputed them in double for every wave).
+struct AttnForm { int tiles, waves; bool multi; };
+inline AttnForm attn_form(int Tkp) {
+    if (Tkp > 1024) return {1, 1, true};
+    const int waves = Tkp <= 256 ? 1 : Tkp <= 512 ? 2 : 4;
+    return {Tkp <= 64 ? 1 : Tkp <= 128 ? 2 : 4, waves, false};
+}
+
 }  // namespace vk
