@@ -94,3 +94,25 @@ def test_make_host_is_deterministic_and_padded():
 def test_bench_refuses_several_gpus():
     r = subprocess.run([sys.executable, str(ROOT / "bench.py"), "--gpus", "2"], capture_output=True, text=True, timeout=120)
     assert r.returncode == 2 and "one GPU" in r.stderr
+
+
+@pytest.mark.parametrize("handle", [0, 0x7f00])
+def test_current_stream_without_the_raw_call(monkeypatch, handle):
+    """torch's raw stream getter is not part of its public interface: the public call serves without it."""
+    import torch
+
+    from vela_amd import gemm as vg
+
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream", raising=False)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: type("S", (), {"cuda_stream": handle})())
+    assert vg.stream_ptr() == (handle or None)
+
+
+def test_current_stream_by_the_raw_call(monkeypatch):
+    import torch
+
+    from vela_amd import gemm as vg
+
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda dev: 0x1000 + dev, raising=False)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 2)
+    assert vg.stream_ptr() == 0x1002

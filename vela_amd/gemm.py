@@ -40,8 +40,11 @@ def ptr(t) -> int | None:
 
 def stream_ptr(stream=None) -> int | None:
     if stream is None:
-        # the raw handle, without building a Stream object for each launch
-        return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()) or None
+        # the raw handle, without building a Stream object for each launch, where this torch has the call
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        if raw is not None:
+            return raw(torch.cuda.current_device()) or None
+        stream = torch.cuda.current_stream()
     if isinstance(stream, int):
         return stream or None
     return stream.cuda_stream or None
