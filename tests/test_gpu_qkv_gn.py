@@ -94,7 +94,7 @@ def test_qkv_row_shifts_and_wide_range():
 
 @pytest.mark.parametrize("variant", [1, 2, 3, 4])
 def test_qkv_ignores_tile_override(variant):
-    """QKV runs on the 128 x 128 tiles whatever variant is forced (src/gemm_hl.cu:358 forces 64 x 64)."""
+    """QKV takes its own tiles (by the size) whatever variant is forced (src/gemm_hl.cu:358 forces 64 x 64)."""
     check_qkv(vg.SRC_I16, 2, 77, K=320, seed=20 + variant, variant=variant)
 
 
