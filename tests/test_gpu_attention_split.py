@@ -22,12 +22,17 @@ SMALL = (EXP >> 8).copy()          # starts at 2^22: r needs more than 32 bits
 def check(B, heads, Tq, Tk, causal, scale=70000, table=EXP, seed=0, big_keys=False):
     r = np.random.default_rng(seed + 1000 * Tq + Tk)
     C = heads * 64
-    Tqp, Tkp = (Tq + 63) // 64 * 64, (Tk + 63) // 64 * 64
     X = [r.normal(0, scale, (B * n, C)).astype(np.int32) for n in (Tq, Tk, Tk)]
     X[0][::5] = (X[0][::5] * 0.01).astype(np.int32)      # other shifts among the rows
     X[1][::7] = (X[1][::7] * 0.02).astype(np.int32)
     if big_keys:
         X[1][1] = 1 << 29                                 # eq + ek > 12 for every query
+    check_rows(X, B, heads, Tq, Tk, causal, table)
+
+
+def check_rows(X, B, heads, Tq, Tk, causal, table=EXP):
+    C = heads * 64
+    Tqp, Tkp = (Tq + 63) // 64 * 64, (Tk + 63) // 64 * 64
     q, k, v = gpu_heads(X[0], B, Tq, C, heads, Tqp), gpu_heads(X[1], B, Tk, C, heads, Tkp), gpu_v(X[2], B, Tk, C, heads, Tkp)
     out = torch.full((B * Tq, C), 0x5a5a5a5a, dtype=torch.int32, device="cuda")
     rm = torch.zeros(B * Tq, dtype=torch.int32, device="cuda")
@@ -110,3 +115,37 @@ def test_dominant_key(gpu):
 def test_one_tile(gpu, Tk, causal, kw):
     """Keys of one tile, in the integer arithmetic and in the general one."""
     check(2, 3, 70, Tk, causal, **kw)
+
+
+@pytest.mark.parametrize("T", [150, 300, 700, 1100])
+@pytest.mark.parametrize("kw", [dict(table=RISING), dict(table=SMALL), dict(big_keys=True)])
+def test_general_form_causal(gpu, T, kw):
+    check(1, 1, T, T, True, **kw)
+
+
+@pytest.mark.parametrize("kw", [dict(), dict(table=SMALL)])
+def test_causal_past_the_staged_keys(gpu, kw):
+    """More keys than the LDS constants hold at a time, causal: queries on both sides of the restaging."""
+    check(1, 1, 4170, 4170, True, **kw)
+
+
+@pytest.mark.parametrize("total", [12, 13])
+@pytest.mark.parametrize("Tk", [20, 77, 200, 400, 1000, 1100])
+def test_dominant_key_by_form(gpu, Tk, total):
+    """test_dominant_key with the shifts held: eq + ek = 12 at most, the last sum of the integer arithmetic (where r =
+    2^32 is taken as 2^32 - 1), and 13, the first of the general one, for every form by the number of keys."""
+    r = np.random.default_rng(Tk)
+    Tq, lo, hi = 33, 1 << 20, (1 << 21) - 1            # shift 6
+    sign = r.choice([-1, 1], 64)
+    Xq, Xk = r.integers(lo, hi, (Tq, 64)) * sign, r.integers(-hi, hi, (Tk, 64))
+    Xk[:, 0] = r.choice([-1, 1], Tk) * r.integers(lo, hi, Tk)
+    top = [0, Tk // 2, Tk - 1][Tk % 3]
+    Xk[top] = hi * sign
+    if total == 13:
+        Xk[(top + 1) % Tk, 3] = hi + 1                 # shift 7
+    eq, ek = oracle.quant_heads(Xq.astype(np.int32), 1, Tq, 64, 1, 64)[2], oracle.quant_heads(Xk.astype(np.int32), 1, Tk, 64, 1, (Tk + 63) // 64 * 64)[2]
+    assert eq[:Tq].min() == eq[:Tq].max() == 6 and eq.max() + ek.max() == total
+    # scores in Q16, a margin of 1 % for the rounding: all but one key 16 e-folds and more below, so that sum E = 2^30
+    S = np.sort((Xq.astype(np.float64) @ Xk.T.astype(np.float64)) / 2**19, axis=1)
+    assert (S[:, -1] - S[:, -2] > 1.01 * 2**20).all() and EXP[0] == 1 << 30
+    check_rows([Xq.astype(np.int32), Xk.astype(np.int32), r.integers(-(2**31), 2**31, (Tk, 64), dtype=np.int64).astype(np.int32)], 1, 1, Tq, Tk, False)
