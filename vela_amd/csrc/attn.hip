@@ -18,9 +18,9 @@
 //   * KW waves share a block's queries and split the keys (KW 64 NT >= Tkp): they exchange row
 //     maxima and sums through LDS and add their partial outputs there. More keys than that (MULTI): one
 //     wave sees all keys and recomputes the scores in each pass.
-//   * 20 vector instructions per pair with the scores kept (37 recomputed), four cycles each when they issue
-//     back to back: that, and the lane permutes of the operands, bound the kernel, not memory (leaving the
-//     loads out gains 2 %).
+//   * Vector instructions bound the kernel, four cycles each when they issue back to back, and the lane permutes of
+//     the operands, not memory (leaving the loads out gains 2 %): by the counters of whole calls 29 per pair with the
+//     scores kept (80 groups of 1024 x 1024), 41 recomputed in each pass (40 groups of 4096 x 4096), MFMAs among them.
 //   * The unsigned-offset terms of the planes ride in the MFMA accumulators' initial values: with q =
 //     256 qh + ql + 128 and likewise k, S = 65536 hh + 256 hl + ll where hl starts at 128 qhs + qls / 2
 //     and ll at 128 ksum (+ 128 when qls is odd).
@@ -372,7 +372,7 @@ __device__ __forceinline__ void attn_body(const AttnArgs& a, const AttnLds& s, i
             w.tile_max(kt, sv[0], m);
         });
     } else {
-if (any) {
+        if (any) {
             // rows loaded PF subtiles ahead, permuted one ahead, scores finished one behind the MFMAs
             typename W::Frag kb[PF], kn;
             typename W::Acc acc;
@@ -416,7 +416,7 @@ if (any) {
             se = W::tile_sum(sv[0], se);
         });
     } else {
-if (any) {
+        if (any) {
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
                 w.tile_exp(w.kt0 + t, sv[t]);
@@ -468,43 +468,43 @@ if (any) {
         }
     } else {
         if (any) {
-        v4i pn_h[NT], pn_l[NT];
-        typename W::Frag vb[PF], vn;   // V rows loaded PF ahead, dimension by dimension, permuted one ahead
-        auto vload = [&](int i) { return w.load_v(tile(i % NT), i / NT); };
+            v4i pn_h[NT], pn_l[NT];
+            typename W::Frag vb[PF], vn;   // V rows loaded PF ahead, dimension by dimension, permuted one ahead
+            auto vload = [&](int i) { return w.load_v(tile(i % NT), i / NT); };
 #pragma unroll
-        for (int i = 0; i < PF; ++i) vb[i] = vload(i);
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            w.tile_p(sv[t], pn_h[t], pn_l[t], psum);
-        }
-        psum += __shfl_xor(psum, 16);
-        psum += __shfl_xor(psum, 32);
-        vn = w.spread(vb[0]);
-        // |O| < 2^31 (the P of a row sum to at most 32768 + Tk / 2 < 2^16), so partial sums may wrap
-#pragma unroll
-        for (int ds = 0; ds < 4; ++ds) {
-            v4i hh = v4i{0, 0, 0, 0}, hl = hh, ll = hh;
+            for (int i = 0; i < PF; ++i) vb[i] = vload(i);
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                const int i = ds * NT + t;
-                const typename W::Frag v = vn;
-                if (i + PF < 4 * NT) vb[i % PF] = vload(i + PF);
-                if (i + 1 < 4 * NT) vn = w.spread(vb[(i + 1) % PF]);
-                W::pv(v, pn_h[t], pn_l[t], hh, hl, ll);
+                w.tile_p(sv[t], pn_h[t], pn_l[t], psum);
             }
-            unsigned O[4];
+            psum += __shfl_xor(psum, 16);
+            psum += __shfl_xor(psum, 32);
+            vn = w.spread(vb[0]);
+            // |O| < 2^31 (the P of a row sum to at most 32768 + Tk / 2 < 2^16), so partial sums may wrap
 #pragma unroll
-            for (int j = 0; j < 4; ++j) O[j] = 128u * unsigned(psum) - ((unsigned(hh[j]) << 16) + (unsigned(hl[j]) << 8) + unsigned(ll[j]));
-            if (KW > 1) {
+            for (int ds = 0; ds < 4; ++ds) {
+                v4i hh = v4i{0, 0, 0, 0}, hl = hh, ll = hh;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) __hip_atomic_fetch_add((LDS_AS unsigned*)s.o + (qw * 64 + 16 * ds + 4 * fg + j) * O_LD + fr, O[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-            } else {
-                int o4[4];
+                for (int t = 0; t < NT; ++t) {
+                    const int i = ds * NT + t;
+                    const typename W::Frag v = vn;
+                    if (i + PF < 4 * NT) vb[i % PF] = vload(i + PF);
+                    if (i + 1 < 4 * NT) vn = w.spread(vb[(i + 1) % PF]);
+                    W::pv(v, pn_h[t], pn_l[t], hh, hl, ll);
+                }
+                unsigned O[4];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) o4[j] = attn_out(double(int(O[j])), ev[16 * ds + 4 * fg + j], am);
-                if (store) *reinterpret_cast<int4*>(orow + 16 * ds + 4 * fg) = make_int4(o4[0], o4[1], o4[2], o4[3]);
+                for (int j = 0; j < 4; ++j) O[j] = 128u * unsigned(psum) - ((unsigned(hh[j]) << 16) + (unsigned(hl[j]) << 8) + unsigned(ll[j]));
+                if (KW > 1) {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) __hip_atomic_fetch_add((LDS_AS unsigned*)s.o + (qw * 64 + 16 * ds + 4 * fg + j) * O_LD + fr, O[j], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                } else {
+                    int o4[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) o4[j] = attn_out(double(int(O[j])), ev[16 * ds + 4 * fg + j], am);
+                    if (store) *reinterpret_cast<int4*>(orow + 16 * ds + 4 * fg) = make_int4(o4[0], o4[1], o4[2], o4[3]);
+                }
             }
-        }
         }
         if (KW > 1) {
             // the summed outputs, four dimensions of a query per thread: 16 lanes share a query
@@ -724,8 +724,8 @@ __global__ void __launch_bounds__(256) quant_heads_pad_kernel(int G, int T, int 
 
 // src/kernels.cu:632-650 (k_quant_v, exponents): ev = row_exp(max |x|) per dimension. row_exp is monotone,
 // so blocks of QV_ROWS rows of a group combine their exponents by an atomic maximum on a cleared ev; the
-// clear also zeroes vsum for the write pass. One block per group scanning all rows, four loads deep, took
-// 267 us of 4096 rows in 40 groups (1 MB a block); in runs of 128 rows the clear and the scan take 11.
+// clear also zeroes vsum for the write pass. One block per group scanning all rows (1 MB a block), four loads deep,
+// was most of the operand's time: 4096 rows in 40 groups 286 us with the write pass, 26 in runs of 128 rows.
 constexpr int QV_ROWS = 128;
 constexpr int QV_ONE = 128;    // keys a block quantises on its own, in one launch in place of three
 __global__ void __launch_bounds__(256) quant_v_clear_kernel(int n, int32_t* __restrict__ ev, long long* __restrict__ vsum) {

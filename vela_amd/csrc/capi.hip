@@ -111,7 +111,8 @@ struct Tiles { int BM, BN; };
 // variant 3 (128 x 256, eight waves) exists for the DMA sources only; the register-staged sources
 // run it as variant 0
 constexpr int NVARIANT = 4;
-constexpr Tiles TILES[NVARIANT + 1] = {{128, 128}, {64, 128}, {128, 64}, {128, 256}, {64, 320}};
+constexpr Tiles TILES[NVARIANT] = {{128, 128}, {64, 128}, {128, 64}, {128, 256}};
+constexpr Tiles tile_of(int variant) { return variant == vk::TILE_X32_WIDE ? Tiles{64, 320} : TILES[variant]; }
 using vk::cdiv;
 using vk::NCU;
 
@@ -264,7 +265,7 @@ int pick_splitk(int variant, int M, int N, int Kp) {
     if (g_splitk > 0) return g_splitk < nK ? g_splitk : nK;
     const SplitRule rule = split_rule(M, N, Kp);
     if (rule == SPLIT_NONE) return 1;
-    const long long tiles = (long long)cdiv(M, TILES[variant].BM) * cdiv(N, TILES[variant].BN);
+    const long long tiles = (long long)cdiv(M, tile_of(variant).BM) * cdiv(N, tile_of(variant).BN);
     long long s = 2LL * NCU / tiles;   // one round of blocks
     if (rule == SPLIT_SMALL && s > 6) s = 6;
     if (s > nK / 16) s = nK / 16;
@@ -327,8 +328,8 @@ ViewWs2 view_ws2(int M, int nout) {
 
 size_t ws_bytes_for(int variant, int M, int N, int splits) {
     if (splits <= 1) return 0;
-    const size_t rows = size_t(cdiv(M, TILES[variant].BM)) * TILES[variant].BM;
-    const size_t cols = size_t(cdiv(N, TILES[variant].BN)) * TILES[variant].BN;
+    const size_t rows = size_t(cdiv(M, tile_of(variant).BM)) * tile_of(variant).BM;
+    const size_t cols = size_t(cdiv(N, tile_of(variant).BN)) * tile_of(variant).BN;
     return size_t(splits) * 2 * rows * cols * 4;
 }
 
@@ -666,8 +667,8 @@ int hl2_impl(void* stream, const VgemmASrc* A, int Mp, int Mreal, const int8_t* 
     if (A->src == VGEMM_SRC_CONV32 && g_variant < 0 && p.C % 64 == 0) variant = 1;
     // int32 rows likewise (K % 4 == 0)
     if (A->src == VGEMM_SRC_X32 && g_variant < 0 && p.K % 4 == 0) variant = x32_wide(epi, p, Kp) ? vk::TILE_X32_WIDE : 1;
-    // whole heads per wave: 128 x 128 tiles, or 64 x 128 ones (int16 rows, int8 planes) while the larger leave
-    // CUs without a block (1024 x 640 x 1920, 120 tiles, 17.2 -> 12.3 us; 240 tiles 18.4 -> 17.4; from 512 tiles on
+    // whole heads per wave: 128 x 128 tiles, or 64 x 128 ones (int16 rows, int8 planes) up to one of the larger per
+    // CU (1024 x 640 x 1920, 120 tiles, 17.2 -> 12.3 us; 240 tiles 18.4 -> 17.4; from 512 tiles on
     // the larger are ahead, 22.2 against 24.4). The reference forces its 64 x 64 tile (src/gemm_hl.cu:358).
     if (epi == VGEMM_EPI_QKV)
         variant = (A->src == VGEMM_SRC_I8 || A->src == VGEMM_SRC_I16) && (long long)cdiv(Mreal, TILES[0].BM) * cdiv(Nreal, TILES[0].BN) <= NCU ? 1 : 0;
@@ -677,9 +678,9 @@ int hl2_impl(void* stream, const VgemmASrc* A, int Mp, int Mreal, const int8_t* 
         const Tiles rt = gn_ref_tile(Mp, Np, Kp, A->src);
         p.gnBM = rt.BM;
         p.gnBN = rt.BN;
-        if (!halo_bm && (TILES[variant].BM % rt.BM || TILES[variant].BN % rt.BN)) variant = 0;
+        if (!halo_bm && (tile_of(variant).BM % rt.BM || tile_of(variant).BN % rt.BN)) variant = 0;
     }
-    const int BM = TILES[variant].BM, BN = TILES[variant].BN;
+    const int BM = tile_of(variant).BM, BN = tile_of(variant).BN;
     p.mtiles = cdiv(Mreal, BM);
     p.ntiles = cdiv(Nreal, BN);
     const int nK = halo_bm ? p.C / 64 : (Kp + 63) / 64;
@@ -853,8 +854,8 @@ int vgemm_i8_run(void* handle, void* stream, const int8_t* A, int lda, long long
     p.Mreal = M; p.Nreal = N; p.Kp = K; p.K = K;
     p.sA = strideA; p.sW = strideW; p.sC = strideC;
     const int variant = g_variant >= 0 && g_variant < NVARIANT ? g_variant : pick_variant_raw(M, N, K);
-    p.mtiles = cdiv(M, TILES[variant].BM);
-    p.ntiles = cdiv(N, TILES[variant].BN);
+    p.mtiles = cdiv(M, tile_of(variant).BM);
+    p.ntiles = cdiv(N, tile_of(variant).BN);
     const int nK = (K + 63) / 64;
     p.ksplit = 1; p.kper = nK;
     p.stride = 1;
@@ -863,7 +864,7 @@ int vgemm_i8_run(void* handle, void* stream, const int8_t* A, int lda, long long
     const VgemmI8Handle* h = static_cast<const VgemmI8Handle*>(handle);
     const long long tiles = (long long)p.mtiles * p.ntiles;
     if (batch == 1 && h->ws && tiles < NCU && nK >= 32 && ldc % 4 == 0 && g_splitk != 1) {
-        const long long rows = (long long)p.mtiles * TILES[variant].BM, cols = (long long)p.ntiles * TILES[variant].BN;
+        const long long rows = (long long)p.mtiles * tile_of(variant).BM, cols = (long long)p.ntiles * tile_of(variant).BN;
         const long long plane = rows * cols * 4;
         long long s = g_splitk > 1 ? g_splitk : std::min<long long>(2LL * NCU / tiles, nK / 16);
         s = std::min<long long>(s, (long long)(h->ws_bytes / size_t(plane)));

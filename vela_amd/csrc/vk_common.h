@@ -33,7 +33,7 @@ constexpr unsigned OOB = 0x80000000u;
 // Third descriptor word of a raw (untyped) buffer resource on gfx9-family GPUs.
 constexpr int RSRC_WORD3 = 0x00020000;
 
-constexpr int TILE_X32_WIDE = 4;   // tile variant of int32 rows, 64 x 320, beyond the ones that can be forced
+constexpr int TILE_X32_WIDE = 16;   // tile variant of int32 rows, 64 x 320, apart from the numbers that vgemm_set_variant takes
 
 struct GemmParams {
     // A operand
