@@ -45,7 +45,8 @@ def test_edges(epi, M, N, K):
 
 @pytest.mark.parametrize("e_max", [0, 6, 11])
 def test_automatic_route(e_max):
-    """3100 x 320 x 2560: 980 tiles of 64x128, the row-stationary kernels with and without shifts."""
+    """3100 x 320 x 2560: 980 tiles of 64x128, the row-stationary kernel without shifts and, with two chunks a block, the tile
+    kernels with them."""
     Case(vg.SRC_I8, 3100, 2560, 320, epi=vg.EPI_GEGLU, seed=5 + e_max, rowmax=True, s_range=(23, 26), e_max=e_max).check(what=f"auto e {e_max}")
 
 
