@@ -63,6 +63,7 @@ def test_int32_rows_on_wide_tiles(rules, M, N, K, wide):
     (1, 2944, 2568, 320, False),     # 16.1 / 17.1 in double
     (1, 4713, 2560, 320, False),     # 24.7 / 25.2, 27.8 in double
     # five K steps whatever Kp is
+    (1, 34188, 640, 128, False),   # 1.13 times in double
     (1, 61568, 72, 64, False), (0, 24576, 512, 64, False), (1, 3136, 2560, 64, False), (1, 10844, 2560, 96, False), (2, 3136, 2560, 64, False),
     # few rows, few tiles
     (0, 16384, 320, 320, False), (1, 1000, 8000, 320, False), (1, 1400, 2560, 320, False),

@@ -45,18 +45,20 @@ inline StripeRanges stripe_ranges(int M, int N) {
 // and 960 64x128 tiles on (below, at 768 tiles, 16384 x 320 x 320 12.3 against 13.4 us on it), where a block has the
 // chunks that pay for its set-up and the grid's rounds of two blocks a CU are filled. The kernel runs five K steps
 // whatever Kp is, so Kp < 128 stays on the tiles but for wide GELU (61568 x 64 x 72 GEGLU 13.3 -> 19.6 us on it,
-// 24576 x 64 x 512 PLAIN 17.2 -> 20.3, 9932 x 96 x 2560 GELU 48.7 -> 37.5). The lines are those of 2500 calls, K 64 to
-// 320 and N 64 to 5120, in the integer form, the one in double (shifts up to 12) and the general one (us; in brackets
-// in double). From 960 columns, where the tile kernels take 128x128 tiles:
+// 24576 x 64 x 512 PLAIN 17.2 -> 20.3, 9932 x 96 x 2560 GELU 48.7 -> 37.5). The lines are those of 4800 calls, K 64 to
+// 320 and N 64 to 5120, in the integer form, the one in double (shifts up to 12) and the general one: those sent here
+// take 0.78 of the tile kernels' time, 0.6 % of them over 1.02 and at most 1.09 (us below; in brackets in double).
+// From 960 columns, where the tile kernels take 128x128 tiles:
 //   GEGLU, one round      three chunks a block   8320 x 320 x 1280 23.5 -> 18.1 (19.7), two: 2944 x 320 x 2568 16.1 -> 16.2 (17.1)
 //   GEGLU, more rounds    four                   6592 x 320 x 2560 35.0 -> 28.7 (32.5), three: 4713 x 320 x 2560 24.7 -> 25.2 (27.8)
 //   PLAIN, GELU           two                    7040 x 320 x 1280 PLAIN 24.3 -> 20.4, 3136 x 320 x 2560 17.3 -> 15.6
 // Below 960 columns:
 //   one round             always                 61568 x 320 x 64 15.9 -> 13.7, 12352 x 320 x 640 18.1 -> 15.2
 //   more rounds           by the share of the rounds' chunk slots that is used: half from five chunks a block on (GELU
-//                         from three), 55 % at four, 70 % at three: 38400 x 320 x 640 GEGLU 44 -> 33.5, 64000 x 320 x
-//                         320 39.4 -> 32.3; less, or two chunks: 14080 x 320 x 640 19.8 -> 20.4 (22.4), 16640 x 320 x 640
-//                         21.9 -> 23.2 (26.1), 61568 x 320 x 72 16.5 -> 20.6
+//                         from three; 60 % at Kp = 128: 34188 x 128 x 640 GEGLU 1.13 times in double at 52 %), 55 % at
+//                         four, 70 % at three: 38400 x 320 x 640 GEGLU 44 -> 33.5, 64000 x 320 x 320 39.4 -> 32.3;
+//                         less, or two chunks: 14080 x 320 x 640 19.8 -> 20.4 (22.4), 16640 x 320 x 640 21.9 -> 23.2
+//                         (26.1), 61568 x 320 x 72 16.5 -> 20.6
 enum ShiftEpi { SHIFT_PLAIN, SHIFT_GEGLU, SHIFT_GELU };
 inline bool stripe_shift_rows(ShiftEpi epi, int M, int N, int Kp) {
     if (M < 1024 || (long long)cdiv(M, 64) * cdiv(N, 128) < 15LL * NCU / 4) return false;
@@ -67,7 +69,7 @@ inline bool stripe_shift_rows(ShiftEpi epi, int M, int N, int Kp) {
     if (N >= 960) return kper >= (epi != SHIFT_GEGLU ? 2 : rounds == 1 ? 3 : 4);
     if (rounds == 1) return true;
     const double used = double(mt * cdiv(N, STRIPE_CH)) / double(rounds * 2 * NCU * kper);
-    if (kper >= (gelu ? 3 : 5)) return used >= 0.5;
+    if (kper >= (gelu ? 3 : 5)) return used >= (gelu || Kp > 128 ? 0.5 : 0.6);
     return (kper == 4 && used >= 0.55) || (kper == 3 && used >= 0.7);
 }
 
