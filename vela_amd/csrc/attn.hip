@@ -725,7 +725,8 @@ __global__ void __launch_bounds__(256) quant_heads_pad_kernel(int G, int T, int 
 // src/kernels.cu:632-650 (k_quant_v, exponents): ev = row_exp(max |x|) per dimension. row_exp is monotone,
 // so blocks of QV_ROWS rows of a group combine their exponents by an atomic maximum on a cleared ev; the
 // clear also zeroes vsum for the write pass. One block per group scanning all rows (1 MB a block), four loads deep,
-// was most of the operand's time: 4096 rows in 40 groups 286 us with the write pass, 26 in runs of 128 rows.
+// was most of the operand's time: 4096 rows in 40 groups 286 us with the write pass, 26 in runs of 128 rows (calls
+// back to back; 127 and 28 by the kernel trace of an attention layer).
 constexpr int QV_ROWS = 128;
 constexpr int QV_ONE = 128;    // keys a block quantises on its own, in one launch in place of three
 __global__ void __launch_bounds__(256) quant_v_clear_kernel(int n, int32_t* __restrict__ ev, long long* __restrict__ vsum) {

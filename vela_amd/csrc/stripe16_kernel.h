@@ -24,9 +24,9 @@
 // chunk's MFMAs, the plane sums folded into one int32 per element (256 Chi + Clo, exact for
 // Kp <= 320) across the barrier. RX instantiations take rows with shifts in the integer form too (the planes
 // the norms and row quantisations write): the multiplier is shifted by the row's e and the offset term added
-// to the sum, two more instructions per requantisation (32768 x 320 x 2560 GEGLU with row shifts: 118 us on
-// the 128x128 tiles, 66-68 here, 62 without shifts). The int64 form (per-row shifts, columns whose constants fail the
-// integer form's bounds, tables outside [0, 65536]) runs a plain loop, a chunk's MFMAs then its
+// to the sum, two more instructions per requantisation (32768 x 320 x 2560 GEGLU with row shifts, repeated calls: 118 us on
+// the 128x128 tiles, 68-73 here, 62 without shifts). The int64 form (columns and shifts past the other
+// forms' bounds, tables outside [0, 65536]) runs a plain loop, a chunk's MFMAs then its
 // outputs element by element.
 #pragma once
 #include "stripe_kernel.h"
